@@ -22,6 +22,7 @@ HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "liboracle.so"
 REF_PATH = HERE / "_ref" / "libbfly_ref.so"
 REFERENCE_TREE = Path("/root/reference")
+REFERENCE_SOURCE = REFERENCE_TREE / "src" / "framework" / "reference.cpp"
 
 _f32p = np.ctypeslib.ndpointer(np.float32, flags="C_CONTIGUOUS")
 _f64p = np.ctypeslib.ndpointer(np.float64, flags="C_CONTIGUOUS")
@@ -40,7 +41,7 @@ APP_MODES = {"ofdm": 0, "radar": 1, "dl": 2}
 def build(with_ref: bool = True) -> None:
     """Compile the C oracle (and, when the reference tree exists, oracle/_ref)."""
     subprocess.run(["make", "-s", "-C", str(HERE), "all"], check=True)
-    if with_ref and REFERENCE_TREE.exists():
+    if with_ref and REFERENCE_SOURCE.exists():
         subprocess.run(["make", "-s", "-C", str(HERE), "ref"], check=True)
 
 
@@ -119,7 +120,7 @@ def ref():
     global _ref
     if _ref is None:
         if not REF_PATH.exists():
-            if REFERENCE_TREE.exists():
+            if REFERENCE_SOURCE.exists():
                 build(with_ref=True)
             if not REF_PATH.exists():
                 return None
