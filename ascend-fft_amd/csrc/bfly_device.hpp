@@ -51,6 +51,18 @@ __device__ __forceinline__ void st_io(float2* p, float2 x) {
     else *p = x;
 }
 
+// Workgroups are dealt to the 8 XCDs in turn.  Within each window of 8 W
+// consecutive ones, gives XCD x the W neighbouring units x W .. x W + W - 1
+// instead of every eighth one, so that units sharing a 128-byte line meet in
+// that XCD's L2 while the 8 XCDs still work on neighbouring units.  A
+// permutation of 0 .. nb - 1 (the last, partial window is dealt the same way
+// in eighths, its remainder as it comes).
+__device__ __forceinline__ uint32_t xcd_window(uint32_t b, uint32_t nb, uint32_t W) {
+    const uint32_t base = b - b % (8u * W), q = b - base, left = nb - base;
+    const uint32_t w = left >= 8u * W ? W : left / 8u;
+    return q < 8u * w ? base + (q & 7u) * w + (q >> 3) : b;
+}
+
 // ------------------------------------------------------------ complex ops
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }

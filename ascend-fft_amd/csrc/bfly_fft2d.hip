@@ -3,21 +3,25 @@
 //
 // X[k1][k2] = sum_{j1, j2} x[j1][j2] W_n1^{j1 k1} W_n2^{j2 k2} is separable:
 // the row pass is the C2C kernels over batch * n1 rows of n2 points; the
-// column pass runs k_cols, which takes C = WG / T adjacent columns per
-// workgroup of WG threads (T = threads per column transform), so every load
-// and store is a run of C consecutive complex values (C * 8 bytes: 128 B at
-// 256-point columns, 512 B at 64).  Column lengths up to 2048 are one
-// k_cols pass (512 / 1024 / 2048 in 512 / 1024 / 1024-thread workgroups);
-// 4096 is split n1 = P * Q = 64 * 64 (four-step along the columns):
+// column pass takes C adjacent columns per workgroup, so that every load and
+// store is a run of C consecutive complex values.  Columns are numbered
+// through the batch, so a group may span two items and no lane idles where
+// the columns per item are few or no multiple of C.  Two kernels:
+//
+//   k_cols       16 points per thread, up to 256-point columns (and few
+//                512-point ones): 256-thread workgroups, C >= 16;
+//   k_cols_wide  32 points per thread (bfly_wide.hpp), 512 to 4096 points in
+//                256 / 512 / 1024-thread workgroups (launch_wide).
+//
+// One pass, so the 2-D transform is two HBM round trips.  Fewer than
+// kOnePassCols 4096-point columns are split n1 = P * Q = 64 * 64 instead
+// (four-step along the columns, more and shorter workgroups):
 //
 //   j1 = Q p + q,  k1 = kp + P kq
 //   Y[Q kp + q][c] = W_n1^{q kp} * FFT_P over p of x[Q p + q][c]   (k_cols, twiddle)
 //   X[kp + P kq][c] = FFT_Q over q of Y[Q kp + q][c]              (k_cols, row map)
 //
-// so the whole transform is two HBM round trips up to n1 = 2048 and three
-// at 4096.  The column transforms use the LDS twiddle tables of the streaming
-// C2C kernels (stockham_lt); the inter-pass twiddle is W_n1^e =
-// A[e mod 64] * B[e / 64] from two LDS tables.
+// with W_n1^e = A[e mod 64] * B[e / 64] from two LDS tables.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -26,24 +30,50 @@
 #include "bfly_kernels.hpp"
 #include "bfly_tables.hpp"
 #include "bfly_units.hpp"
+#include "bfly_wide.hpp"
 
 namespace {
 
 using namespace bfly_dev;
 
 // Addressing of one column pass.  A batch item of `item` elements holds
-// `mats` matrices; matrix m of item b reads rows at in + b*item +
-// m*in_mstride (row pitch in_rstride) and writes at out + b*item +
-// m*out_mstride (row pitch out_rstride); columns are `ncols` wide, walked
-// by `groups` workgroups of C columns.
+// `mats` matrices of `ncols` columns; matrix m of item b reads rows at
+// in + b*item + m*in_mstride (row pitch in_rstride) and writes at
+// out + b*item + m*out_mstride (row pitch out_rstride).  Columns are numbered
+// f = (b*mats + m)*ncols + column, `total` of them.
 struct ColView {
     uint64_t item;
     uint64_t in_mstride, out_mstride;
     uint32_t in_rstride, out_rstride;
-    uint32_t ncols, groups, mats;
+    uint32_t ncols, mats, total;
     uint32_t col_div;  // twiddle pass: q = column / col_div
+    int temporal;      // see line_aligned
+    uint32_t win;      // units per XCD window (set by the launcher)
 };
 
+// Rows that start on 128-byte lines: a run of 16 or more columns then covers
+// whole lines and takes the streaming hint (512 x 1024 x 32: 51.0 us against
+// 53.3 without it).  Other rows share every line with the neighbouring
+// columns' workgroup, which the L2 serves and merges only without the hint
+// (512 x 1001 x 24, windows of 8: 50.8 us against 76.4 with it).
+bool line_aligned(const void* in, const void* out, uint32_t ncols) {
+    return ncols % 16 == 0 && (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 128 == 0;
+}
+
+// Units per XCD window (xcd_window) of the column kernels.  Sweep 1 / 2 / 4 /
+// 8 / 16 / 64 of the 16-point kernel: 512 x 1001 x 24 66.6 / 58.3 / 53.1 /
+// 50.8 / 50.4 / 54.3 us, 256 x 1024 x 64 55.3 / 55.1 / 54.4 / 51.3 / 48.9 us
+// (1 .. 16), 64 x 1001 x 200 53.5 / 49.2 / 46.0 / 44.6 / 42.6 / 42.6.
+constexpr uint32_t kColWindow = 16;
+
+// 4096-point columns from which one pass is used (4096 x 64 x 16, 1024 of
+// them: 18.5 us against 27.9 in two passes, 2-D 4096 x 256 x 4 41.0 against
+// 45.8; 512 of them: 17.8 against 14.1).
+constexpr uint32_t kOnePassCols = 1024;
+
+// One column group per workgroup: C = WG / T adjacent columns, 16 points per
+// thread.  Bound by HBM (run lengths of C columns); columns up to 256 points,
+// and 512-point ones in few groups (column_pass).
 template <int I, int DIR, bool TW, int WG = bfly_plan::kBlock>
 __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ wab,
@@ -60,188 +90,280 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
     __shared__ float2 ltw[LT::LEN];
     __shared__ float2 wt[TW ? 128 : 1];
     const int tid = threadIdx.x;
-    // the column plan's tables: [its pass tables | A | B] as in the local C2C table
-    c2c_lds_tw<I, WG>(ltw, tw, tw + bfly_plan::stage_twiddle_len(I), tid);
-    if constexpr (TW)
-        for (int i = tid; i < 128; i += WG) wt[i] = wab[i];
+    // the column plan's tables, [its pass tables | A | B] as in the local C2C
+    // table: fetched ahead of the columns, parked in LDS behind their loads
+    C2cLdsTwFetch<I, WG> tabs;
+    tabs.fetch(tw, tw + bfly_plan::stage_twiddle_len(I), tid);
     const int c = tid % C, t = tid / C;
-    // groups narrower than a 128-byte line (C = 8) share each line with the
-    // next group: workgroups are dealt to the 8 XCDs in turn, so within each
-    // window of 16 the pair of groups 2x, 2x+1 goes to XCD x (dealt 8 apart)
-    // and meets in its L2, while the 8 XCDs still work on adjacent columns
-    const uint32_t nb = gridDim.x, b0 = blockIdx.x;
-    const uint32_t blk = (C < 16 && (b0 | 15) < nb) ? (b0 & ~15u) | ((b0 & 7u) << 1) | ((b0 >> 3) & 1u) : b0;
-    const uint32_t g = blk % cv.groups;
-    const uint64_t mi = blk / cv.groups;
-    const uint64_t b = mi / cv.mats, m = mi % cv.mats;
-    const uint32_t col = g * C + c;
-    const bool active = col < cv.ncols;
+    const uint32_t blk = xcd_window(blockIdx.x, gridDim.x, cv.win), f = blk * C + c;
+    const bool active = f < cv.total;
+    uint32_t mi, col;  // matrix and column of this lane
+    if (cv.ncols % C == 0) {  // whole groups: one division per workgroup
+        const uint32_t groups = cv.ncols / C;
+        mi = blk / groups;
+        col = (blk - mi * groups) * C + c;
+    } else {
+        mi = f / cv.ncols;
+        col = f - mi * cv.ncols;
+    }
+    uint32_t b = mi, m = 0;
+    if (cv.mats > 1) {
+        b = mi / cv.mats;
+        m = mi - b * cv.mats;
+    }
     const float2* src = in + b * cv.item + m * cv.in_mstride + col;
     float2 v[P];
+    auto load = [&](auto nt) {
 #pragma unroll
-    for (int mm = 0; mm < P / R0; mm++)
+        for (int mm = 0; mm < P / R0; mm++)
 #pragma unroll
-        for (int r = 0; r < R0; r++)
-            v[mm * R0 + r] = active ? ld_stream(&src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))])
-                                    : make_float2(0.f, 0.f);
+            for (int r = 0; r < R0; r++)
+                v[mm * R0 + r] =
+                    active ? ld_io<decltype(nt)::value>(&src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))])
+                           : make_float2(0.f, 0.f);
+    };
+    if (cv.temporal) load(std::false_type{});
+    else load(std::true_type{});
+    tabs.park(ltw, tid);
+    if constexpr (TW)
+        for (int i = tid; i < 128; i += WG) wt[i] = wab[i];
     // the transform's first LDS exchange orders the table writes before any read
     run_plan_lt<I, T, DIR, LX_PAD>(v, lds + c * STRIDE, 0, ltw, ltw + LT::NLO, ltw + LT::NLO + LT::NHI, t,
                                    std::make_index_sequence<PL::NRAD>{});
     if (!active) return;
     float2* dst = out + b * cv.item + m * cv.out_mstride + col;
     const uint32_t q = TW ? col / cv.col_div : 0u;
-#pragma unroll
-    for (int mm = 0; mm < P / RL; mm++)
-#pragma unroll
-        for (int r = 0; r < RL; r++) {
-            const int k = t + mm * T + r * (L / RL);
-            float2 x = v[mm * RL + r];
-            if constexpr (TW) {
-                const uint32_t e = q * (uint32_t)k;  // < n1 <= 4096
-                const float2 a = wt[e & 63], w = wt[64 + (e >> 6)];
-                x = cmul_tw<DIR>(x, make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x));
-            }
-            st_stream(&dst[(uint64_t)cv.out_rstride * k], x);
-        }
-}
-
-// Streaming form of k_cols (no twiddle, every column group full): a
-// resident grid walks the units (C-column groups of every matrix, in the
-// one-shot grid's order) with the next unit's loads in flight through the
-// current unit's passes.  Loads and stores go through per-unit raw buffer
-// descriptors (zero records past the last unit, so no branch guards the
-// prefetch) with the per-row offset in the scalar operand, and the tables
-// are staged once per workgroup.  Same per-column arithmetic as k_cols, so
-// the same bits.  Used where one workgroup fills a CU (1024-point columns,
-// 139 KiB of LDS), which otherwise loads, computes and stores in turn.
-template <int I, int DIR, int WG>
-__global__ __launch_bounds__(WG) void k_cols_stream(const float2* __restrict__ in, float2* __restrict__ out,
-                                                    const float2* __restrict__ tw, ColView cv, uint32_t units,
-                                                    uint32_t in_span, uint32_t out_span) {
-    using PL = PlanOf<I>;
-    using LT = C2cLdsTw<I>;
-    constexpr int L = PL::N, T = PL::T, C = WG / T;
-    constexpr int R0 = PL::R0, RL = PL::RL, P = PL::P;
-    constexpr int STRIDE = lds_len(L) + 1;
-    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-    __shared__ float2 lds[C * STRIDE];
-    __shared__ float2 ltw[LT::LEN];
-    const int tid = threadIdx.x;
-    c2c_lds_tw<I, WG>(ltw, tw, tw + bfly_plan::stage_twiddle_len(I), tid);
-    // (the first unit's first LDS exchange orders these writes before the reads)
-    const int c = tid % C, t0 = tid / C;
-    // element offsets of unit u's first column, input and output side
-    auto base = [&](uint32_t u, uint64_t& oin, uint64_t& oout) {
-        const uint32_t g = u % cv.groups, mi = u / cv.groups;
-        const uint32_t b = mi / cv.mats, m = mi % cv.mats;
-        oin = (uint64_t)b * cv.item + (uint64_t)m * cv.in_mstride + (uint64_t)g * C;
-        oout = (uint64_t)b * cv.item + (uint64_t)m * cv.out_mstride + (uint64_t)g * C;
-    };
-    auto load_unit = [&](float2 (&v)[P], uint32_t u, bool valid, int t) {
-        uint64_t oin, oout;
-        base(u, oin, oout);
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float2*>(in + oin), (short)0,
-                                                          valid ? (int)in_span : 0, 0x00020000);
-        const uint32_t voff = ((uint32_t)t * cv.in_rstride + (uint32_t)c) * 8u;
-#pragma unroll
-        for (int mm = 0; mm < P / R0; mm++)
-#pragma unroll
-            for (int r = 0; r < R0; r++) {
-                const uint32_t soff = (uint32_t)(mm * T + r * (L / R0)) * cv.in_rstride * 8u;
-                v[mm * R0 + r] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 2));
-            }
-    };
-    float2 cur[P], nxt[P];
-    auto step = [&](uint32_t u) {
-        int t = t0;  // opaque per-step thread index (see k_r2c_stream)
-        asm volatile("" : "+v"(t));
-        const uint32_t un = u + gridDim.x;
-        load_unit(nxt, un < units ? un : u, un < units, t);
-        run_plan_lt<I, T, DIR, LX_PAD>(cur, lds + c * STRIDE, 0, ltw, ltw + LT::NLO, ltw + LT::NLO + LT::NHI, t,
-                                       std::make_index_sequence<PL::NRAD>{});
-        uint64_t oin, oout;
-        base(u, oin, oout);
-        const auto os = __builtin_amdgcn_make_buffer_rsrc(out + oout, (short)0, (int)out_span, 0x00020000);
-        const uint32_t voff = ((uint32_t)t * cv.out_rstride + (uint32_t)c) * 8u;
+    auto store = [&](auto nt) {
 #pragma unroll
         for (int mm = 0; mm < P / RL; mm++)
 #pragma unroll
             for (int r = 0; r < RL; r++) {
-                const uint32_t soff = (uint32_t)(mm * T + r * (L / RL)) * cv.out_rstride * 8u;
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, cur[mm * RL + r]), os, voff, soff, 2);
+                const int k = t + mm * T + r * (L / RL);
+                float2 x = v[mm * RL + r];
+                if constexpr (TW) {
+                    const uint32_t e = q * (uint32_t)k;  // < n1 <= 4096
+                    const float2 a = wt[e & 63], w = wt[64 + (e >> 6)];
+                    x = cmul_tw<DIR>(x, make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x));
+                }
+                st_io<decltype(nt)::value>(&dst[(uint64_t)cv.out_rstride * k], x);
             }
-        // the stores issue before the register copy waits for the prefetch
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < P; i++) cur[i] = nxt[i];
     };
-    uint32_t u = blockIdx.x;  // the grid never exceeds the unit count
-    load_unit(cur, u, true, t0);
-    step(u);
-    for (u += gridDim.x; u < units; u += gridDim.x) step(u);
+    if (cv.temporal) store(std::false_type{});
+    else store(std::true_type{});
 }
 
-template <int I, bool TW, int WG = bfly_plan::kBlock>
-hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const float2* wab, ColView cv,
-                       uint64_t batch, int sign, hipStream_t s) {
-    constexpr int C = WG / PlanOf<I>::T;
-    cv.groups = (cv.ncols + C - 1) / C;
-    const uint64_t blocks = batch * cv.mats * cv.groups;
-    if (blocks == 0 || blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    // 1024-point columns: the streaming form when every group is full, a
-    // unit's span fits a buffer descriptor and there is a unit for every
-    // resident slot (2-D 1024x1024 x16: 110.4 -> 106.4 us, 1024x128 x128:
-    // 95.6 -> 91.7; at 512 and 256 points, where two or more workgroups
-    // share a CU, it measured 0.5-2 % slower)
-    if constexpr (!TW && PlanOf<I>::N == 1024 && C >= 16) {
-        const uint64_t in_span = ((uint64_t)(PlanOf<I>::N - 1) * cv.in_rstride + C) * sizeof(float2);
-        const uint64_t out_span = ((uint64_t)(PlanOf<I>::N - 1) * cv.out_rstride + C) * sizeof(float2);
-        if (cv.ncols % C == 0 && in_span < (1ull << 31) && out_span < (1ull << 31)) {
-            static bfly_kern::ResidentCache rc[2];
-            const void* f = sign < 0 ? reinterpret_cast<const void*>(&k_cols_stream<I, -1, WG>)
-                                     : reinterpret_cast<const void*>(&k_cols_stream<I, 1, WG>);
-            const int fit = bfly_kern::resident(rc[sign < 0 ? 0 : 1], f, WG);
-            if (fit > 0 && blocks >= (uint64_t)fit) {
-                if (sign < 0)
-                    hipLaunchKernelGGL((k_cols_stream<I, -1, WG>), dim3((unsigned)fit), dim3(WG), 0, s, in, out, tw,
-                                       cv, (uint32_t)blocks, (uint32_t)in_span, (uint32_t)out_span);
-                else
-                    hipLaunchKernelGGL((k_cols_stream<I, 1, WG>), dim3((unsigned)fit), dim3(WG), 0, s, in, out, tw,
-                                       cv, (uint32_t)blocks, (uint32_t)in_span, (uint32_t)out_span);
-                return hipGetLastError();
-            }
-        }
+// Plans of the wide column kernel: the second pass's twiddles come from its
+// own LDS table, the third pass's from the two-level tables.
+template <int L>
+struct ColPlan;
+template <> struct ColPlan<512> { static constexpr int R0 = 32, R1 = 16, R2 = 1; };
+template <> struct ColPlan<1024> { static constexpr int R0 = 32, R1 = 32, R2 = 1; };
+template <> struct ColPlan<2048> { static constexpr int R0 = 16, R1 = 4, R2 = 32; };
+template <> struct ColPlan<4096> { static constexpr int R0 = 16, R1 = 8, R2 = 32; };
+
+// W_L^m, m < L, from the column table of L.
+template <int L>
+__device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, const float2* __restrict__ wab, int m) {
+    if constexpr (L == 512) {  // last pass of 16 16 2: W^k at [256 + 2 k + 1], k < 256
+        const float2 w = tc[256 + 2 * (m & 255) + 1];
+        return m & 256 ? make_float2(-w.x, -w.y) : w;
+    } else if constexpr (L == 1024) {  // 16 16 4: W^k at [256 + 4 k + 1], quarter turns beyond
+        const float2 w = tc[256 + 4 * (m & 255) + 1];
+        const int q = m >> 8;
+        return q == 0 ? w : q == 1 ? make_float2(w.y, -w.x) : q == 2 ? make_float2(-w.x, -w.y) : make_float2(-w.y, w.x);
+    } else if constexpr (L == 2048) {  // 16 16 8: W^{4 k} at [256 + 8 k + 4], k < 256; here m is a multiple of 32
+        const float2 w = tc[256 + 8 * ((m & 1023) / 4) + 4];
+        return m & 1024 ? make_float2(-w.x, -w.y) : w;
+    } else {
+        const float2 a = wab[m & 63], b = wab[64 + (m >> 6)];
+        return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
     }
+}
+
+// One group of C = 32 WG / L columns per workgroup, 32 points per thread.
+// HBM-bound: one read and one write of every value, in runs of C columns; the
+// exchanges hold one component at a time, so 16384 points take 70 KiB of LDS
+// and two 512-thread workgroups share a CU, where the 16-point kernel's one
+// (139 KiB) loaded, computed and stored in turn.  1024 points take two passes
+// (32 32) instead of three, and 4096 points fit one workgroup at all (two
+// kernels and a third HBM round trip before).  Measured, 16-point kernels ->
+// this one: 1024 x 1024 x 16 59.3 -> 49.0 us (5.5 TB/s), 2048 x 1024 x 8 83.7
+// -> 57.7, 4096 x 1024 x 4 112.3 -> 68; rows that do not start on lines
+// (windows and hints below included): 512 x 1001 x 24 98.6 -> 47.6, 1024 x
+// 1001 x 12 98.4 -> 52.9, 2048 x 999 x 6 120 -> 54, 4096 x 333 x 9 91.5 -> 73.
+template <int L, int DIR, int WG>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_cols_wide(
+    const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tc,
+    const float2* __restrict__ wab, uint32_t ncols, uint32_t total, int stream_in,
+    int stream_out, uint32_t win) {
+    using P = ColPlan<L>;
+    constexpr int T = L / kWide, C = WG / T, LO = 64, HI = L / LO;
+    // columns lie 32 / C banks apart (mod 64), so that the C columns and the
+    // 32 / C consecutive points of a half-wave's access hit 32 banks
+    constexpr int SH = C >= 32 ? 1 : 32 / C;
+    constexpr int STRIDE = lds_len(L) + (SH - lds_len(L) % 64 + 64) % 64;
+    constexpr int T1 = P::R0 * P::R1;
+    __shared__ float lds[C * STRIDE];
+    __shared__ float2 tab[T1 + (P::R2 > 1 ? LO + HI : 0)];
+    const int tid = threadIdx.x;
+    const int c = tid % C;
+    int t = tid / C;
+    // columns are numbered through the batch (f = item * ncols + column)
+    const uint32_t f = xcd_window(blockIdx.x, gridDim.x, win) * C + c;
+    const uint32_t fr = f < total ? f : total - 1;  // past the end: reads the last column again
+    const uint64_t at = (uint64_t)(fr / ncols) * L * ncols + fr % ncols;
+    const float2* src = in + (at + (uint64_t)t * ncols);
+    float2 v[kWide];
+    auto load = [&](auto nt) {
+#pragma unroll
+        for (int m = 0; m < kWide / P::R0; m++)
+#pragma unroll
+            for (int r = 0; r < P::R0; r++)
+                v[m * P::R0 + r] = ld_io<decltype(nt)::value>(src + (uint64_t)(m * T + r * (L / P::R0)) * ncols);
+    };
+    if (stream_in) load(std::true_type{});
+    else load(std::false_type{});
+    // the tables, behind the columns' loads (ahead of them they held the
+    // loads back: 2048 x 1024 x 4 27.5 -> 30.3 us)
+    const float2 *t1 = tab, *tlo = tab + T1, *thi = tlo + LO;
+    for (int i = tid; i < T1; i += WG) tab[i] = col_root<L>(tc, wab, (i / P::R0) * (i % P::R0) * (L / T1));
+    if constexpr (P::R2 > 1) {
+        const float2* ab = L == 4096 ? wab : tc + bfly_plan::stage_twiddle_len(bfly_plan::plan_index(L));
+        for (int i = tid; i < LO + HI; i += WG) tab[T1 + i] = ab[i];
+    }
+    if constexpr (P::R2 > 1) {
+        stockham_wide<L, T, DIR, LO, P::R0, 1, P::R0, P::R1, P::R2>(v, lds + c * STRIDE, tlo, thi, t1, t);
+    } else {
+        stockham_wide<L, T, DIR, LO, P::R0, 1, P::R0, P::R1>(v, lds + c * STRIDE, tlo, thi, t1, t);
+    }
+    if (f >= total) return;
+    constexpr int RL = P::R2 > 1 ? P::R2 : P::R1;
+    asm volatile("" : "+v"(t));
+    float2* dst = out + (at + (uint64_t)t * ncols);
+    auto store = [&](auto nt) {
+#pragma unroll
+        for (int m = 0; m < kWide / RL; m++)
+#pragma unroll
+            for (int r = 0; r < RL; r++)
+                st_io<decltype(nt)::value>(dst + (uint64_t)(m * T + r * (L / RL)) * ncols, v[m * RL + r]);
+    };
+    if (stream_out) store(std::true_type{});
+    else store(std::false_type{});
+}
+
+template <int L, int WG>
+hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, const float2* wab, uint32_t ncols,
+                            uint32_t total, bool aligned, int sign, hipStream_t s) {
+    constexpr uint32_t C = WG / (L / kWide);
+    const uint32_t blocks = (uint32_t)(((uint64_t)total + C - 1) / C);
+    // Access hints and windows (kColWindow: why windows; line_aligned: why
+    // other rows stay without hints).  Whole-line rows take the streaming
+    // hint on the input: read into the L2s without it, the lines of a buffer
+    // that another kernel writes next (the 2-D transform's workspace) made
+    // that kernel's writes slow (2-D 1024 x 256 x 8 18.2 us against 23.2).
+    // Outputs of runs under a line (2048 and 4096 points) are merged in the
+    // L2 without the hint (4096 x 1024 x 4: 66.7 us against 76), except at
+    // 2048 points and 512 threads (2-D 2048 x 256 x 4: 22.5 against 24.1);
+    // so are 1024-point ones in one round of workgroups (1024 x 256 x 32:
+    // 26.9 against 29.1).
+    const int in_hint = aligned;
+    const int out_hint = aligned && (L == 512 || (L == 1024 && (WG < 1024 || blocks >= 512)) || (L == 2048 && WG == 512));
+    const uint32_t win = !aligned ? 32 : WG == 1024 ? (L == 1024 && ncols <= 256 ? 64 : 32) : WG == 512 && L < 2048 ? 32 : 4;
     if (sign < 0)
-        hipLaunchKernelGGL((k_cols<I, -1, TW, WG>), dim3((unsigned)blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, total,
+                           in_hint, out_hint, win);
     else
-        hipLaunchKernelGGL((k_cols<I, 1, TW, WG>), dim3((unsigned)blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, total,
+                           in_hint, out_hint, win);
     return hipGetLastError();
 }
 
-template <bool TW>
-hipError_t cols(uint32_t len, const float2* in, float2* out, const float2* tw, const float2* wab, ColView cv,
-                uint64_t batch, int sign, hipStream_t s) {
+// Picks the wide kernel's workgroup: the largest that still gives every CU
+// one.  A larger one takes longer runs (256 bytes at 1024 points and 1024 threads)
+// and, at 1024 threads, the whole LDS of a CU, which pays where a run is
+// whole lines (1024 x 1024 x 16: 48.7 us against 55.7 at 512 threads; 2048 x
+// 1024 x 8: 55.0 against 75.9) or, at 4096 points, too short anyway (4096 x
+// 1024 x 4: 69.3 against 85.5; 4096 x 333 x 4: 34.5 against 39.7); other rows
+// run best at 512 threads, two workgroups to a CU (2048 x 999 x 6: 55.1
+// against 62.6).  Few columns: 256 threads (1024 x 64 x 4: 6.9 us against
+// 10.4 at 512 threads; 2048 x 100 x 8: 11.5 against 13.9).
+template <int L>
+hipError_t launch_wide(const float2* in, float2* out, const float2* tc, const float2* wab, uint32_t ncols,
+                       uint32_t total, bool aligned, bool rows_behind, int sign, hipStream_t s) {
+    constexpr uint32_t kCus = 256;
+    // (right behind the 2-D transform's row pass, narrow matrices run better
+    // at 512 threads: 2-D 1024 x 128 x 128 90.4 us against 95.1, where the
+    // column pass by itself takes 61.1 against 51.8)
+    if constexpr (L >= 1024)
+        if ((aligned || L == 4096) && !(L == 1024 && rows_behind && ncols < 256) && total >= kCus * (32768u / L))
+            return launch_cols_wide<L, 1024>(in, out, tc, wab, ncols, total, aligned, sign, s);
+    // (2048 points: from half that, 2-D 2048 x 256 x 4 22.5 us against 26.8)
+    if (L == 4096 || total >= kCus * (16384u / L) / (L == 2048 && aligned ? 2 : 1))
+        return launch_cols_wide<L, 512>(in, out, tc, wab, ncols, total, aligned, sign, s);
+    if constexpr (L < 4096) return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
+    return hipErrorInvalidValue;
+}
+
+template <int I, bool TW, int WG = bfly_plan::kBlock>
+hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const float2* wab, ColView cv, int sign,
+                       hipStream_t s) {
+    constexpr uint32_t C = WG / PlanOf<I>::T;
+    const uint32_t blocks = (uint32_t)(((uint64_t)cv.total + C - 1) / C);
+    // whole-line rows in a round of workgroups or less: as dealt (the split's
+    // first pass at 4096 x 64 x 4 5.4 us against 6.6)
+    cv.win = cv.temporal || blocks >= 1024 ? kColWindow : 1;
+    if (sign < 0)
+        hipLaunchKernelGGL((k_cols<I, -1, TW, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+    else
+        hipLaunchKernelGGL((k_cols<I, 1, TW, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+    return hipGetLastError();
+}
+
+// The column pass; `rows_behind`: of a 2-D transform whose row pass has just
+// written `in`.
+hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols, uint32_t batch, int sign,
+                              const float* table_cols, void* work, bool rows_behind, hipStream_t s) {
+    const float2* i2 = reinterpret_cast<const float2*>(in);
+    float2* o2 = reinterpret_cast<float2*>(out);
+    const float2* tc = reinterpret_cast<const float2*>(table_cols);
+    const bfly_host::Fft2dLayout L = bfly_host::fft2d_layout(n1);
+    const uint64_t item = (uint64_t)n1 * ncols, total = (uint64_t)ncols * batch;
+    // the guards keep batch * n1 * ncols / 16 below 2^31, so column and
+    // workgroup counts fit 32 bits
+    if (total == 0 || total > 0x7fffffffull) return hipErrorInvalidValue;
+    const uint32_t F = (uint32_t)total;
+    const bool al = line_aligned(in, out, ncols);
     constexpr auto idx = bfly_plan::plan_index;
-    // the twiddle pass runs the first factor of a split length (32 or 64)
-    if constexpr (!TW)
-        if (len == 16) return launch_cols<idx(16), TW>(in, out, tw, wab, cv, batch, sign, s);
-    switch (len) {
-        case 32: return launch_cols<idx(32), TW>(in, out, tw, wab, cv, batch, sign, s);
-        case 64: return launch_cols<idx(64), TW>(in, out, tw, wab, cv, batch, sign, s);
-        case 128: return launch_cols<idx(128), TW>(in, out, tw, wab, cv, batch, sign, s);
-        case 256: return launch_cols<idx(256), TW>(in, out, tw, wab, cv, batch, sign, s);
+    // (16 and 32 points: runs of 2 and 1 KiB are mostly whole lines however
+    // the rows start: 16 x 1000 x 700 32.6 us with the hint, 34.7 without)
+    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, al || n1 <= 32 ? 0 : 1, 1};
+    const float2* t1 = tc + L.p_table;
+    switch (n1) {
+        case 16: return launch_cols<idx(16), false>(i2, o2, t1, nullptr, cv, sign, s);
+        case 32: return launch_cols<idx(32), false>(i2, o2, t1, nullptr, cv, sign, s);
+        case 64: return launch_cols<idx(64), false>(i2, o2, t1, nullptr, cv, sign, s);
+        case 128: return launch_cols<idx(128), false>(i2, o2, t1, nullptr, cv, sign, s);
+        case 256: return launch_cols<idx(256), false>(i2, o2, t1, nullptr, cv, sign, s);
+        case 512:
+            // whole-line rows in fewer column groups than the wide kernel
+            // needs to fill the chip: 512 x 64 x 4 5.7 us against 6.3, 512 x
+            // 64 x 128 11.6 against 12.7 (512 x 64 x 256: 26.4 against 23.1)
+            if (al && F < 12288) return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, sign, s);
+            return launch_wide<512>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
+        case 1024: return launch_wide<1024>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
+        case 2048: return launch_wide<2048>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
         default: break;
     }
-    // 512 / 1024 / 2048-point columns in one pass: 16 / 16 / 8 columns per
-    // workgroup in 512 / 1024 / 1024-thread workgroups (70 / 139 / 139 KiB
-    // of LDS)
-    if constexpr (!TW) {
-        if (len == 512) return launch_cols<idx(512), TW, 512>(in, out, tw, wab, cv, batch, sign, s);
-        if (len == 1024) return launch_cols<idx(1024), TW, 1024>(in, out, tw, wab, cv, batch, sign, s);
-        if (len == 2048) return launch_cols<idx(2048), TW, 1024>(in, out, tw, wab, cv, batch, sign, s);
-    }
-    return hipErrorInvalidValue;
+    const float2* wab = tc + L.wab;
+    if (F >= kOnePassCols) return launch_wide<4096>(i2, o2, t1, wab, ncols, F, al, rows_behind, sign, s);
+    // P-point pass with the twiddle: in -> ws; Q-point pass with the row map: ws -> out
+    float2* ws = reinterpret_cast<float2*>(work);
+    const uint32_t qn = L.q * ncols;
+    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, line_aligned(in, ws, qn) ? 0 : 1, 1};
+    hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, wab, a, sign, s);
+    if (e != hipSuccess) return e;
+    const ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, L.p, qn * batch, 1, line_aligned(ws, out, ncols) ? 0 : 1, 1};
+    return launch_cols<idx(64), false>(ws, o2, tc + L.q_table, nullptr, b, sign, s);
 }
 
 }  // namespace
@@ -250,38 +372,22 @@ namespace bfly_kern {
 
 hipError_t columns(const float* in, float* out, uint32_t n1, uint32_t ncols, uint32_t batch, int sign,
                    const float* table_cols, void* work, hipStream_t s) {
-    const float2* i2 = reinterpret_cast<const float2*>(in);
-    float2* o2 = reinterpret_cast<float2*>(out);
-    float2* ws = reinterpret_cast<float2*>(work);
-    const float2* tc = reinterpret_cast<const float2*>(table_cols);
-    const bfly_host::Fft2dLayout L = bfly_host::fft2d_layout(n1);
-    const uint64_t item = (uint64_t)n1 * ncols;
-    if (L.q == 1) {
-        ColView cv{item, 0, 0, ncols, ncols, ncols, 0, 1, 1};
-        return cols<false>(n1, i2, o2, tc + L.p_table, nullptr, cv, batch, sign, s);
-    }
-    // P-point pass with the twiddle: in -> ws; Q-point pass with the row map: ws -> out
-    const uint32_t qn = L.q * ncols;
-    ColView a{item, 0, 0, qn, qn, qn, 0, 1, ncols};
-    hipError_t e = cols<true>(L.p, i2, ws, tc + L.p_table, tc + L.wab, a, batch, sign, s);
-    if (e != hipSuccess) return e;
-    ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, 0, L.p, 1};
-    return cols<false>(L.q, ws, o2, tc + L.q_table, nullptr, b, batch, sign, s);
+    return column_pass(in, out, n1, ncols, batch, sign, table_cols, work, false, s);
 }
 
 hipError_t fft2d(const float* in, float* out, uint32_t n1, uint32_t n2, uint32_t batch, int sign,
                  const float* table_rows, const float* table_cols, void* work, hipStream_t s) {
     // the row pass takes the C2C kernel the library picks for (n2, batch * n1)
     const int rows = bfly_host::auto_variant(n2, batch * n1);
-    if (bfly_host::fft2d_layout(n1).q == 1) {
+    if (n1 < 4096 || (uint64_t)n2 * batch >= kOnePassCols) {
         // rows in -> work, columns work -> out
         float* w = static_cast<float*>(work);
         hipError_t e = c2c(in, w, n2, batch * n1, sign, rows, table_rows, nullptr, s);
-        return e != hipSuccess ? e : columns(w, out, n1, n2, batch, sign, table_cols, nullptr, s);
+        return e != hipSuccess ? e : column_pass(w, out, n1, n2, batch, sign, table_cols, nullptr, true, s);
     }
     // rows in -> out, columns out -> work -> out
     hipError_t e = c2c(in, out, n2, batch * n1, sign, rows, table_rows, nullptr, s);
-    return e != hipSuccess ? e : columns(out, out, n1, n2, batch, sign, table_cols, work, s);
+    return e != hipSuccess ? e : column_pass(out, out, n1, n2, batch, sign, table_cols, work, true, s);
 }
 
 }  // namespace bfly_kern

@@ -119,17 +119,45 @@ struct C2cLdsTw {
     static constexpr int LEN = NLO + NHI + NT1;
 };
 
-// Fills `buf` (C2cLdsTw<I>::LEN entries) from the plan's pass tables `tw` and
-// `ab` = [W_N^j, j < NLO | W_N^{NLO j}, j < NHI] in device memory.  The
-// caller synchronises before the tables are read.
+// Entry i of the tables, from the plan's pass tables `tw` and `ab` =
+// [W_N^j, j < NLO | W_N^{NLO j}, j < NHI] in device memory.
+template <int I>
+__device__ __forceinline__ float2 c2c_lds_tw_entry(const float2* __restrict__ tw, const float2* __restrict__ ab, int i) {
+    using L = C2cLdsTw<I>;
+    if (kPlans[I].nrad == 1 || i < L::NLO + L::NHI) return ab[i];
+    const int j = i - L::NLO - L::NHI;  // [r 16 + k] from the pass table's [k R1 + r]
+    return tw[(j % bfly_plan::kPoints) * L::R1 + j / bfly_plan::kPoints];
+}
+template <int I>
+constexpr int c2c_lds_tw_len() { return C2cLdsTw<I>::NLO + C2cLdsTw<I>::NHI + (kPlans[I].nrad > 1 ? C2cLdsTw<I>::NT1 : 0); }
+
+// Fills `buf` (C2cLdsTw<I>::LEN entries).  The caller synchronises before
+// the tables are read.
 template <int I, int WG>
 __device__ __forceinline__ void c2c_lds_tw(float2* buf, const float2* __restrict__ tw,
                                            const float2* __restrict__ ab, int tid) {
-    using L = C2cLdsTw<I>;
-    for (int i = tid; i < L::NLO + L::NHI; i += WG) buf[i] = ab[i];
-    if constexpr (kPlans[I].nrad > 1)
-        for (int i = tid; i < L::NT1; i += WG) buf[L::NLO + L::NHI + (i % L::R1) * bfly_plan::kPoints + i / L::R1] = tw[i];
+    for (int i = tid; i < c2c_lds_tw_len<I>(); i += WG) buf[i] = c2c_lds_tw_entry<I>(tw, ab, i);
 }
+
+// The same in two halves, for a kernel that issues its data loads in
+// between: the tables' latency then overlaps the data's.
+template <int I, int WG>
+struct C2cLdsTwFetch {
+    static constexpr int LEN = c2c_lds_tw_len<I>(), K = (LEN + WG - 1) / WG;
+    float2 e[K];
+    __device__ __forceinline__ void fetch(const float2* __restrict__ tw, const float2* __restrict__ ab, int tid) {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int i = tid + k * WG;
+            e[k] = c2c_lds_tw_entry<I>(tw, ab, i < LEN ? i : LEN - 1);  // no branch around the load
+        }
+    }
+    __device__ __forceinline__ void park(float2* buf, int tid) const {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (tid + k * WG < LEN) buf[tid + k * WG] = e[k];
+    }
+};
 
 template <int I, int DIR, int WG>
 __device__ __forceinline__ void c2c_unit_lt(const float2* __restrict__ in, float2* __restrict__ out,
