@@ -290,7 +290,10 @@ int bfly_c2c_traced(const float* in, float* out, uint32_t n, uint32_t batch, int
         if (!events[i]) return BFLY_ERR_SHAPE;
     if (int g = bfly_host::check_execute(BFLY_KIND_C2C, sign, in, out, n, batch, table, work, variant))
         return g;
-    if (variant == BFLY_VARIANT_AUTO) variant = bfly_host::auto_variant(n, batch);
+    // a traced chain (32768 and 65536 points) times its two launches whatever
+    // AUTO runs untraced
+    if (variant == BFLY_VARIANT_AUTO)
+        variant = launches == 2 ? bfly_host::auto_variant(n, batch) : bfly_host::auto_kernel(n, batch);
     const bool uses_work = launches == 2;
     if (!bfly_host::disjoint(BFLY_KIND_C2C, in, out, uses_work ? work : nullptr, n, batch, 0, 0))
         return BFLY_ERR_SHAPE;
@@ -307,7 +310,7 @@ static int c2c_checked(const float* in, float* out, uint32_t n, uint32_t batch, 
     if (int g = bfly_host::check_execute(BFLY_KIND_C2C, sign, in, out, n, batch, table, work, variant))
         return g;
     if (variant < BFLY_VARIANT_AUTO || variant > BFLY_VARIANT_LAST) return BFLY_ERR_SHAPE;
-    if (variant == BFLY_VARIANT_AUTO) variant = bfly_host::auto_variant(n, batch);
+    if (variant == BFLY_VARIANT_AUTO) variant = bfly_host::auto_kernel(n, batch);
     const bool uses_work = bfly_host::needs_work(BFLY_KIND_C2C, n, batch, variant);
     if (!bfly_host::disjoint(BFLY_KIND_C2C, in, out, uses_work ? work : nullptr, n, batch, 0, 0))
         return BFLY_ERR_SHAPE;
@@ -322,9 +325,10 @@ int bfly_c2c_ex(const float* in, float* out, uint32_t n, uint32_t batch, int sig
 int bfly_c2c_scaled(const float* in, float* out, uint32_t n, uint32_t batch, int sign, float scale,
                     const float* table, void* work, void* stream) {
     if (!std::isfinite(scale)) return BFLY_ERR_SHAPE;
-    // validate n before it picks a variant; check_execute repeats it
-    if (!bfly_supported(BFLY_KIND_C2C, n)) return BFLY_ERR_SHAPE;
-    return c2c_checked(in, out, n, batch, sign, bfly_host::scaled_variant(n, batch), table, work, stream, scale);
+    // the variant whose last store applies the scale (AUTO above 4096; see
+    // bfly_host::scaled_variant)
+    const int variant = n <= (uint32_t)bfly_plan::kMaxLocalN ? BFLY_VARIANT_STREAM_LT : BFLY_VARIANT_AUTO;
+    return c2c_checked(in, out, n, batch, sign, variant, table, work, stream, scale);
 }
 
 int bfly_c2c(const float* in, float* out, uint32_t n, uint32_t batch, int sign,

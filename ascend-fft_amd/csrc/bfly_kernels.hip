@@ -996,6 +996,7 @@ hipError_t c2c(const float* in, float* out, uint32_t n, uint32_t batch, int sign
         default: break;
     }
     const bfly_host::TableLayout L = bfly_host::table_layout(0, n);
+    if (variant == bfly_host::kVariantWide) return c2c_wide(i2, o2, tw + L.extra, n, batch, sign, scale, n, n, s);
     if (variant == BFLY_VARIANT_STREAM_LT && n <= (uint32_t)bfly_plan::kMaxSingleN) {
         const float2 *ts = tw + L.single, *wN = tw + L.extra;
         switch (n) {
@@ -1063,6 +1064,9 @@ hipError_t c2c_rows(const float* in, uint64_t idist, float* out, uint64_t odist,
     const bfly_host::TableLayout L = bfly_host::table_layout(0, n);
     const float2 *t1 = tw + L.stage0, *t2 = tw + L.stage1, *wN = tw + L.extra;
     float2* ws = reinterpret_cast<float2*>(work);
+    // (32768: the kernel AUTO picks, so that contiguous rows equal bfly_c2c)
+    if (bfly_host::auto_kernel(n, batch) == bfly_host::kVariantWide)
+        return c2c_wide(i2, o2, wN, n, batch, sign, 1.0f, idist, odist, s);
     switch (n) {
         case 32768:
             return launch_long<idx(128), idx(256)>(i2, o2, ws, t1, t2, wN, batch, sign, s, nullptr, 1.0f, idist, odist);

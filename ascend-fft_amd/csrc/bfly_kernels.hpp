@@ -21,8 +21,7 @@ int resident(ResidentCache& cache, const void* kernel, int block);
 // `mid`, when given, is recorded on `s` between the two launches of the
 // four-step chain (unused by the one-launch paths).  `scale` multiplies
 // every output in the final store; the LDS-twiddle streaming kernels
-// (BFLY_VARIANT_STREAM_LT, and 8192 / 16384 under AUTO) and the four-step
-// chain apply it, the other variants require 1.
+// (BFLY_VARIANT_STREAM_LT), kVariantWide and the four-step chain apply it, the other variants require 1.
 // Batched C2C over rows `idist` / `odist` complex values apart (>= n):
 // the LDS-twiddle streaming kernel for n 16..16384, the four-step chain
 // (contiguous workspace `work`) for 32768 / 65536; `table` as for c2c.
@@ -30,6 +29,11 @@ hipError_t c2c_rows(const float* in, uint64_t idist, float* out, uint64_t odist,
                     int sign, const float* table, void* work, hipStream_t s);
 hipError_t c2c(const float* in, float* out, uint32_t n, uint32_t batch, int sign, int variant,
                const float* table, void* work, hipStream_t s, hipEvent_t mid = nullptr, float scale = 1.0f);
+// C2C of n = 8192, 16384 or 32768 with the 32-point core, one transform per
+// workgroup (bfly_wide.hip); `wN` is the W_n^m table, distances in complex
+// values.
+hipError_t c2c_wide(const float2* in, float2* out, const float2* wN, uint32_t n, uint32_t batch, int sign,
+                    float scale, uint64_t idist, uint64_t odist, hipStream_t s);
 // variant: BFLY_VARIANT_PLAIN (one-shot grid), BFLY_VARIANT_STREAM or
 // BFLY_VARIANT_STREAM_LT; `adjoint` runs the transform's adjoint (R2C: the
 // C2R's adjoint weighting of the bins; C2R: the R2C's).

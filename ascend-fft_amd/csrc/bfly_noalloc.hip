@@ -66,7 +66,7 @@ int bfly_noalloc_prepare(void) {
 int bfly_c2c_noalloc(const float* in, float* out, uint32_t n, uint32_t batch, int sign, const float* table,
                      void* stream) {
     const bool known = bfly_supported(BFLY_KIND_C2C, n) && batch;
-    const int variant = known ? bfly_host::auto_variant(n, batch) : BFLY_VARIANT_AUTO;
+    const int variant = known ? bfly_host::auto_kernel(n, batch) : BFLY_VARIANT_AUTO;
     const bool chain = known && bfly_host::needs_work(BFLY_KIND_C2C, n, batch, variant);
     // the argument guards of bfly_c2c first (a non-null stand-in for the
     // workspace they would otherwise ask the caller for) ...

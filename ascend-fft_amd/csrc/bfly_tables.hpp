@@ -77,8 +77,13 @@ int check_fft2d(int sign, const void* in, const void* out, uint32_t n1, uint32_t
 // Mode-truncated real transforms: 1 <= bins <= n/2+1, stride (floats) even
 // and at least 2*bins.
 bool bins_ok(uint32_t n, uint32_t bins, uint32_t stride);
-// The variant BFLY_VARIANT_AUTO resolves to for a C2C of (n, batch).
+// The public variant nearest to what BFLY_VARIANT_AUTO runs for a C2C of
+// (n, batch): it decides the workspace and the launch count callers see.
 int auto_variant(uint32_t n, uint32_t batch);
+// The kernel BFLY_VARIANT_AUTO runs for a C2C of (n, batch): auto_variant's,
+// or kVariantWide (bfly_wide.hip), which has no public id.
+constexpr int kVariantWide = 64;
+int auto_kernel(uint32_t n, uint32_t batch);
 // The variant BFLY_VARIANT_AUTO resolves to for a real transform of (n, batch).
 int auto_real_variant(uint32_t n, uint32_t batch);
 // Guards and shape of one bfly_host_pipelined call (shared by the HIP library
@@ -93,8 +98,9 @@ struct PipeShape {
 int check_pipelined(int kind, int sign, int variant, const void* host_in, const void* host_out, uint32_t n,
                     uint32_t batch, const void* table, const void* dev_in, const void* dev_out, const void* work,
                     uint32_t chunk_rows, PipeShape* shape);
-// The variant bfly_c2c_scaled runs: one whose last store applies the scale
-// (the LDS-twiddle streaming kernel up to n = 8192, AUTO's choice above).
+// The public variant nearest to what bfly_c2c_scaled runs, one whose last
+// store applies the scale: the LDS-twiddle streaming kernel up to n = 4096,
+// AUTO's choice above.
 int scaled_variant(uint32_t n, uint32_t batch);
 
 // Guards of bfly_mode_mix: op 0..2, non-null 8-byte aligned operands, every

@@ -194,7 +194,7 @@ BFLY_API int bfly_c2c_inv(const float* in, float* out, uint32_t n, uint32_t batc
  * counterpart (its C2C is unnormalised and only C2R applies 1/n,
  * src/ascendc/fft_real.cpp:167-267); it serves callers of the public inverse
  * who want numpy's norm="backward" / "ortho" / "forward" conventions.
- * Runs the LDS-twiddle streaming kernels up to n = 8192 and AUTO's choice
+ * Runs the LDS-twiddle streaming kernels up to n = 4096 and AUTO's choice
  * above, so the result equals fl(scale * bfly_c2c_ex(..., variant)) bit for
  * bit for that variant.  `scale` must be finite (else BFLY_ERR_SHAPE);
  * `work` as for bfly_c2c. */
@@ -251,8 +251,8 @@ BFLY_API int bfly_c2c_columns(const float* in, float* out, uint32_t n, uint32_t 
  * to bfly_c2c_ex(..., BFLY_VARIANT_STREAM_LT, ...) bit for bit); 32768 and
  * 65536 run the four-step chain, whose column pass reads the padded input
  * and row pass writes the padded output, through `work` of
- * bfly_workspace_bytes(BFLY_KIND_C2C, n, batch) bytes (with idist = odist
- * = n equal to bfly_c2c bit for bit).  No counterpart
+ * bfly_workspace_bytes(BFLY_KIND_C2C, n, batch) bytes, or AUTO's kernel of
+ * 32768 points (with idist = odist = n equal to bfly_c2c bit for bit).  No counterpart
  * in the reference: non-contiguous contracts are future work there
  * (config/test_matrix.json:94-99, 106 "fft2d-and-strides"). */
 BFLY_API int bfly_c2c_rows(const float* in, uint64_t idist, float* out, uint64_t odist, uint32_t n, uint32_t batch,
@@ -307,7 +307,11 @@ BFLY_API int bfly_c2c_traced(const float* in, float* out, uint32_t n, uint32_t b
  *                        prefetches each workgroup's next transforms
  * For n <= 4096 FOUR_STEP means PLAIN.  At 8192 / 16384, PLAIN and
  * STREAM_LT run one workgroup per transform (one-shot / streaming) and the
- * other ids the one-shot form; above 16384 every id runs four-step. */
+ * other ids the one-shot form; above 16384 every id runs four-step.  AUTO
+ * runs a kernel of its own, one transform per workgroup of n/32 threads, at
+ * 8192 from 128 transforms, at 16384 from 256 and at 32768 above 128 (there
+ * the workspace is asked for all the same, and bfly_c2c_launches and
+ * bfly_c2c_traced report and time the four-step chain). */
 #define BFLY_VARIANT_AUTO 0
 #define BFLY_VARIANT_PLAIN 1
 #define BFLY_VARIANT_STREAM 2
