@@ -444,10 +444,20 @@ constexpr bool kTwPowers = N != 8192;
 // `t1` holds the second pass's own table in LDS, transposed to [r Ns + k]
 // (Ns = the first radix) so that the lanes of a wave, whose k are
 // consecutive, read consecutive banks: one read per twiddle there; later
-// passes combine the two-level tables.
-template <int N, int P, int T, int DIR, int LX, int Ns, int R, int... Rest>
+// passes combine the two-level tables, or take the third pass's twiddles from
+// `lw` (lt_last_twiddles), which a kernel that walks a batch fills once.
+struct NoKeptTwiddles {
+    static constexpr bool kept = false;
+};
+// The third pass's twiddles of one thread, [m R + r].
+struct KeptTwiddles {
+    static constexpr bool kept = true;
+    float2 w[bfly_plan::kPoints];
+};
+
+template <int N, int P, int T, int DIR, int LX, class LW, int Ns, int R, int... Rest>
 __device__ __forceinline__ void stockham_lt(float2 (&v)[P], float2* lds, int rb, const float2* tlo,
-                                            const float2* thi, const float2* t1, int t) {
+                                            const float2* thi, const float2* t1, int t, const LW& lw) {
     constexpr int M = P / R;
     if constexpr (Ns > 1) {
 #pragma unroll
@@ -456,6 +466,9 @@ __device__ __forceinline__ void stockham_lt(float2 (&v)[P], float2* lds, int rb,
             if constexpr (Ns == bfly_plan::kPoints) {
 #pragma unroll
                 for (int r = 1; r < R; r++) v[m * R + r] = cmul_tw<DIR>(v[m * R + r], t1[r * Ns + k]);
+            } else if constexpr (LW::kept) {
+#pragma unroll
+                for (int r = 1; r < R; r++) v[m * R + r] = cmul_tw<DIR>(v[m * R + r], lw.w[m * R + r]);
             } else if constexpr (kTwPowers<N>) {
                 float2 w[R];
                 tw_powers<N, R>(w, tlo, thi, k * (N / (Ns * R)));
@@ -489,8 +502,44 @@ __device__ __forceinline__ void stockham_lt(float2 (&v)[P], float2* lds, int rb,
             for (int r = 0; r < R2; r++) v[m * R2 + r] = lds[lx_rat<LX, N / R2>(rbase, r)];
         }
         __syncthreads();
-        stockham_lt<N, P, T, DIR, LX, Ns * R, Rest...>(v, lds, rb, tlo, thi, t1, t);
+        stockham_lt<N, P, T, DIR, LX, LW, Ns * R, Rest...>(v, lds, rb, tlo, thi, t1, t, lw);
     }
+}
+
+// Fills `lw` for thread t, as stockham_lt forms the twiddles.
+template <int N, int T, int R>
+__device__ __forceinline__ void lt_keep_twiddles(KeptTwiddles& lw, const float2* tlo, const float2* thi, int t) {
+    static_assert(kTwPowers<N>, "tables combined by tw_powers");
+    constexpr int P = bfly_plan::kPoints, Ns = N / R;
+#pragma unroll
+    for (int m = 0; m < P / R; m++) {
+        float2 w[R];
+        tw_powers<N, R>(w, tlo, thi, (t + m * T) & (Ns - 1));
+#pragma unroll
+        for (int r = 1; r < R; r++) lw.w[m * R + r] = w[r];
+    }
+}
+
+// The rest of stockham_lt once the first pass's butterflies (radix R, v[m R +
+// r]) are done: its exchange and the passes <R2, Rest...>.
+template <int N, int P, int T, int DIR, int LX, class LW, int R, int R2, int... Rest>
+__device__ __forceinline__ void stockham_lt_after_first(float2 (&v)[P], float2* lds, int rb, const float2* tlo,
+                                                        const float2* thi, const float2* t1, int t, const LW& lw) {
+#pragma unroll
+    for (int m = 0; m < P / R; m++) {
+        const int wb = lx_wbase<LX, 1>(rb, (t + m * T) * R);
+#pragma unroll
+        for (int r = 0; r < R; r++) lds[lx_wat<LX, 1>(wb, r)] = v[m * R + r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < P / R2; m++) {
+        const int rbase = lx_rbase<LX, N / R2>(rb, t + m * T);
+#pragma unroll
+        for (int r = 0; r < R2; r++) v[m * R2 + r] = lds[lx_rat<LX, N / R2>(rbase, r)];
+    }
+    __syncthreads();
+    stockham_lt<N, P, T, DIR, LX, LW, R, R2, Rest...>(v, lds, rb, tlo, thi, t1, t, lw);
 }
 
 }  // namespace bfly_dev

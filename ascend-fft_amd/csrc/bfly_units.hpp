@@ -42,12 +42,20 @@ __device__ __forceinline__ void run_plan_rt(float2 (&v)[bfly_plan::kPoints], flo
     stockham_rt<kPlans[I].n, bfly_plan::kPoints, T, DIR, LX, 1, kPlans[I].rad[S]...>(v, lds, rb, tr, t);
 }
 
-template <int I, int T, int DIR, int LX, size_t... S>
+template <int I, int T, int DIR, int LX, size_t... S, class LW = NoKeptTwiddles>
 __device__ __forceinline__ void run_plan_lt(float2 (&v)[bfly_plan::kPoints], float2* lds, int rb,
                                             const float2* tlo, const float2* thi, const float2* t1, int t,
-                                            std::index_sequence<S...>) {
-    stockham_lt<kPlans[I].n, bfly_plan::kPoints, T, DIR, LX, 1, kPlans[I].rad[S]...>(v, lds, rb, tlo, thi,
-                                                                                     t1, t);
+                                            std::index_sequence<S...>, const LW& lw = LW{}) {
+    stockham_lt<kPlans[I].n, bfly_plan::kPoints, T, DIR, LX, LW, 1, kPlans[I].rad[S]...>(v, lds, rb, tlo, thi,
+                                                                                     t1, t, lw);
+}
+
+template <int I, int T, int DIR, int LX, size_t... S, class LW = NoKeptTwiddles>
+__device__ __forceinline__ void run_plan_lt_after_first(float2 (&v)[bfly_plan::kPoints], float2* lds, int rb,
+                                                        const float2* tlo, const float2* thi, const float2* t1,
+                                                        int t, std::index_sequence<S...>, const LW& lw = LW{}) {
+    stockham_lt_after_first<kPlans[I].n, bfly_plan::kPoints, T, DIR, LX, LW, kPlans[I].rad[S]...>(v, lds, rb, tlo, thi,
+                                                                                            t1, t, lw);
 }
 
 template <int I, int T, size_t... S>
@@ -209,16 +217,23 @@ struct RealTwGlobal {
     __device__ __forceinline__ float2 w(int k) const { return wn[k]; }
 };
 
-template <int I>
+template <int I, class LW = NoKeptTwiddles>
 struct RealTwLds {
     const float2* tlo;  // W_M^j, j < 64
     const float2* thi;  // W_M^{64 j}, j < M / 64
     const float2* t1;   // second pass's table, [r 16 + k]
     const float2* wlo;  // W_n^j, j < 64
     const float2* whi;  // W_n^{64 j}, 64 j <= n / 2
+    LW lw{};            // the third pass's twiddles, if kept in registers
     template <int T, int DIR>
     __device__ __forceinline__ void fft(float2 (&v)[bfly_plan::kPoints], float2* L, int t) const {
-        run_plan_lt<I, T, DIR, LX_PAD>(v, L, 0, tlo, thi, t1, t, std::make_index_sequence<kPlans[I].nrad>{});
+        run_plan_lt<I, T, DIR, LX_PAD>(v, L, 0, tlo, thi, t1, t, std::make_index_sequence<kPlans[I].nrad>{}, lw);
+    }
+    // the passes after the first butterfly's arithmetic (its exchange on)
+    template <int T, int DIR>
+    __device__ __forceinline__ void fft_after_first(float2 (&v)[bfly_plan::kPoints], float2* L, int t) const {
+        run_plan_lt_after_first<I, T, DIR, LX_PAD>(v, L, 0, tlo, thi, t1, t,
+                                                   std::make_index_sequence<kPlans[I].nrad>{}, lw);
     }
     __device__ __forceinline__ float2 w(int k) const {
         const float2 a = wlo[k & 63], b = whi[k >> 6];
@@ -261,7 +276,7 @@ __device__ __forceinline__ RealTwLds<I> real_lds_tw(float2* buf, const float2* _
             whi[i - 128 - M / 64 - 16 * R1] = wn[64 * (i - 128 - M / 64 - 16 * R1)];
         }
     }
-    return RealTwLds<I>{tlo, thi, t1, wlo, whi};
+    return RealTwLds<I>{tlo, thi, t1, wlo, whi, {}};
 }
 
 // ------------------------------------------------------------------ R2C
@@ -569,6 +584,162 @@ __device__ __forceinline__ void c2r_finish(float2 (&q)[bfly_plan::kPoints + 1], 
         }
     __syncthreads();
     tws.template fft<T, 1>(v, L, t);
+    if (tr >= batch) return;
+    float2* dst = reinterpret_cast<float2*>(out + tr * (uint64_t)(2 * M));
+#pragma unroll
+    for (int m = 0; m < P / RL; m++)
+#pragma unroll
+        for (int r = 0; r < RL; r++) {
+            const float2 z = v[m * RL + r];
+            st_io<(T >= 16)>(&dst[t + m * T + r * (M / RL)], make_float2(z.x * scale, z.y * scale));
+        }
+}
+
+// The same source with the third pass's twiddles of transform thread t kept
+// in registers (three-pass plans; shorter ones have none to keep).  The tables
+// must be in LDS and synchronised.
+template <int I>
+using RealKept = std::conditional_t<kPlans[I].nrad == 3, KeptTwiddles, NoKeptTwiddles>;
+template <int I>
+__device__ __forceinline__ RealTwLds<I, RealKept<I>> real_keep(const RealTwLds<I>& s, int t) {
+    RealTwLds<I, RealKept<I>> k{s.tlo, s.thi, s.t1, s.wlo, s.whi, {}};
+    if constexpr (RealKept<I>::kept)
+        lt_keep_twiddles<kPlans[I].n, PlanOf<I>::T, kPlans[I].rad[2]>(k.lw, s.tlo, s.thi, t);
+    return k;
+}
+
+// ------------------------------------------------ mode-truncated spectra
+// A truncated R2C stores only its first kout bins.  Up to kout = M / RL (RL =
+// the last pass's radix) they need Z[k] and Z[M - k] of the first and the
+// last of RL equal parts of the spectrum, that is outputs 0 and RL - 1 of
+// each last-pass butterfly: the compiler drops the others' arithmetic, and
+// only two values per butterfly are parked.  Same arithmetic as r2c_finish
+// for the bins it stores.  Ends with LDS reads in flight (see r2c_finish).
+template <int I>
+constexpr bool kTruncR2c = PlanOf<I>::N >= 128 && PlanOf<I>::RL >= 4;
+template <int I, int WG, class TWS>
+__device__ __forceinline__ void r2c_modes_finish(float2 (&v)[bfly_plan::kPoints], float* __restrict__ out,
+                                                 const TWS& tws, uint32_t batch, uint32_t kout, uint32_t ostride,
+                                                 uint32_t g, float2* lds, int tid, bool adj) {
+    using PL = PlanOf<I>;
+    constexpr int M = PL::N, T = PL::T, B = WG / T, RL = PL::RL, P = PL::P, S = M / RL;
+    const int bl = tid / T, t = tid % T;
+    const uint64_t tr = (uint64_t)g * B + bl;
+    float2* L = lds + bl * lds_len(M);
+    tws.template fft<T, -1>(v, L, t);
+    float2* Lm = L + lds_len(S);
+#pragma unroll
+    for (int m = 0; m < P / RL; m++) {
+        L[lds_idx(t + m * T)] = v[m * RL];
+        Lm[lds_idx(t + m * T)] = v[m * RL + RL - 1];
+    }
+    __syncthreads();
+    if (tr >= batch) return;
+    float2* dst = reinterpret_cast<float2*>(out + tr * (uint64_t)ostride);
+#pragma unroll
+    for (int i = 0; i < S / T; i++) {
+        const int k = t + i * T;
+        if (k < (int)kout) {
+            // Z[M - k] is entry S - k of the last part; Z[M] = Z[0]
+            const float2 a = L[lds_idx(k)];
+            const float2 b = k ? Lm[lds_idx(S - k)] : a;
+            const float2 e = make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y));
+            const float2 o = make_float2(0.5f * (a.y + b.y), -0.5f * (a.x - b.x));
+            const float2 wo = cmul_tw<-1>(o, tws.w(k));
+            float2 x = cadd(e, wo);
+            if (adj) {
+                const float f = k == 0 ? 0.5f / (float)M : 1.0f / (float)M;
+                x = make_float2(x.x * f, k == 0 ? 0.f : x.y * f);
+            }
+            st_io<(T >= 16)>(&dst[k], x);
+        }
+    }
+}
+
+// A truncated C2R reads only bins k < kin.  Up to kin = NZ T (T = M / 16, NZ
+// = 2 or 4) the inputs Z'[k] of the first radix-16 butterfly are zero but for
+// its NZ first and NZ last ones, each made from one bin: bin k for k < NZ T,
+// bin M - k for k > M - NZ T.  Every thread loads its own, so nothing is
+// staged in LDS.  q[i] = bin t + i T, q[NZ + i] = bin (i + 1) T - t (zero at
+// or above kin).
+template <int I, int WG, int NZ>
+__device__ __forceinline__ void c2r_modes_load(float2 (&q)[2 * NZ], const float* __restrict__ in, uint32_t batch,
+                                               uint32_t kin, uint32_t istride, uint32_t g, int tid) {
+    using PL = PlanOf<I>;
+    constexpr int T = PL::T, B = WG / T;
+    const int bl = tid / T, t = tid % T;
+    const uint64_t tr = (uint64_t)g * B + bl;
+    // rows past the batch and bins past kin re-read bin 0 of a real row and
+    // are masked: no branch around the loads
+    const float2* src = reinterpret_cast<const float2*>(in + (tr < batch ? tr : 0) * (uint64_t)istride);
+#pragma unroll
+    for (int i = 0; i < 2 * NZ; i++) {
+        const int k = i < NZ ? t + i * T : (i - NZ + 1) * T - t;
+        const bool ok = k < (int)kin;
+        const float2 x = ld_io<(T >= 16)>(&src[ok ? k : 0]);
+        q[i] = make_float2(ok ? x.x : 0.f, ok ? x.y : 0.f);
+    }
+}
+
+// First radix-16 butterfly of the pruned input (r < NZ and r >= 16 - NZ of
+// v[] set): column n2 of its 4 x 4 form holds r = n2 (if n2 < NZ) and r = 12
+// + n2 (if n2 >= 4 - NZ) only.  Equal to dft<16> with zeros elsewhere, up to
+// the sign of zeros.
+template <int NZ, int DIR>
+__device__ __forceinline__ void dft16_edges(float2 (&v)[16]) {
+    static_assert(NZ == 2 || NZ == 4, "two or four edge inputs");
+    float2 y[16];
+#pragma unroll
+    for (int n2 = 0; n2 < 4; n2++) {
+        const bool lo = n2 < NZ, hi = n2 >= 4 - NZ;
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++) {
+            float2 c;
+            if (lo && hi) c = cadd(v[n2], rot16<DIR>(v[12 + n2], 12 * k1));  // quarter turns
+            else if (lo) c = v[n2];
+            else c = rot16<DIR>(v[12 + n2], 12 * k1);
+            y[4 * k1 + n2] = rot16<DIR>(c, n2 * k1);
+        }
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 4; k1++) {
+        float2 c[4];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; n2++) c[n2] = y[4 * k1 + n2];
+        dft4<DIR>(c);
+#pragma unroll
+        for (int k2 = 0; k2 < 4; k2++) v[k1 + 4 * k2] = c[k2];
+    }
+}
+
+// Pre-twiddle of the edge inputs, pruned first pass, the other passes, reals
+// scaled and stored (the steps of c2r_compute).  `adj` as there.  Starts by
+// writing `lds` after the first pass; its exchanges end synchronised.
+template <int I, int WG, int NZ, class TWS>
+__device__ __forceinline__ void c2r_modes_compute(const float2 (&q)[2 * NZ], float* __restrict__ out, const TWS& tws,
+                                                  uint32_t batch, float scale, uint32_t g, float2* lds, int tid,
+                                                  bool adj) {
+    using PL = PlanOf<I>;
+    constexpr int M = PL::N, T = PL::T, B = WG / T, RL = PL::RL, P = PL::P;
+    static_assert(PL::R0 == 16 && P == 16, "one radix-16 butterfly per thread in the first pass");
+    const int bl = tid / T, t = tid % T;
+    const uint64_t tr = (uint64_t)g * B + bl;
+    float2 v[P];
+#pragma unroll
+    for (int i = 0; i < NZ; i++) {
+        float2 a = q[i];
+        if (i == 0 && t == 0) {  // bin 0: real; it has no partner (kin <= M / 2)
+            a.y = 0.f;
+            if (adj) a.x *= 2.f;
+        }
+        const float2 wa = cmul_tw<1>(a, tws.w(t + i * T));  // W_n^{-k} d
+        v[i] = make_float2(a.x - wa.y, a.y + wa.x);
+        const float2 b = q[NZ + i], d = make_float2(-b.x, b.y);
+        const float2 wb = cmul_tw<1>(d, tws.w(t + (15 - i) * T));
+        v[15 - i] = make_float2(b.x - wb.y, wb.x - b.y);
+    }
+    dft16_edges<NZ, 1>(v);
+    tws.template fft_after_first<T, 1>(v, lds + bl * lds_len(M), t);
     if (tr >= batch) return;
     float2* dst = reinterpret_cast<float2*>(out + tr * (uint64_t)(2 * M));
 #pragma unroll
