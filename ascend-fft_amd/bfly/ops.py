@@ -18,8 +18,15 @@ from . import _lib
 _tables: dict = {}
 
 
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+def _stream(t: torch.Tensor) -> int:
+    """Handle of torch's current stream on the tensor's device.  Read raw (the
+    call that generated kernels launch with): building a torch.cuda.Stream
+    object around it costs 1.9 us, the raw read 0.1, of a call whose launch
+    takes 3.8."""
+    device = t.get_device()
+    if device < 0:
+        raise ValueError(f"expected a device tensor, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def supported(kind: int, n: int) -> bool:
@@ -59,20 +66,20 @@ def _check_device(t: torch.Tensor, name: str) -> None:
 
 def c2c_raw(x: torch.Tensor, out: torch.Tensor, n: int, batch: int, sign: int = -1,
             work: torch.Tensor | None = None, scale: float | None = None) -> None:
-    """bfly_c2c on interleaved float32 buffers (no allocation except tables);
-    bfly_c2c_scaled when `scale` is given."""
+    """bfly_c2c on complex64 or interleaved float32 buffers (no allocation
+    except tables); bfly_c2c_scaled when `scale` is given."""
     lib = _lib.hip()
     tab = table(_lib.KIND_C2C, n, x.device)
-    if work is None and lib.bfly_workspace_bytes(_lib.KIND_C2C, n, batch):
+    if work is None:
         work = workspace(_lib.KIND_C2C, n, batch, x.device)
     wp = work.data_ptr() if work is not None else None
     if scale is None:
-        rc = lib.bfly_c2c(x.data_ptr(), out.data_ptr(), n, batch, sign, tab.data_ptr(), wp, _stream(x.device))
+        rc = lib.bfly_c2c(x.data_ptr(), out.data_ptr(), n, batch, sign, tab.data_ptr(), wp, _stream(x))
         if rc:
             _lib.check(rc, f"bfly_c2c(n={n}, batch={batch}, sign={sign})")
     else:
         rc = lib.bfly_c2c_scaled(x.data_ptr(), out.data_ptr(), n, batch, sign, scale, tab.data_ptr(), wp,
-                                 _stream(x.device))
+                                 _stream(x))
         if rc:
             _lib.check(rc, f"bfly_c2c_scaled(n={n}, batch={batch}, sign={sign}, scale={scale})")
 
@@ -101,22 +108,22 @@ def c2c(x: torch.Tensor, sign: int = -1, norm: str | None = None, *, scale: floa
         raise ValueError("give norm or scale, not both")
     _check_device(x, "x")
     if x.dtype == torch.complex64:
+        if x.is_conj():
+            torch.view_as_real(x)  # raises: the memory holds the conjugate
         n = x.shape[-1]
-        xf = torch.view_as_real(x)
+        batch = x.numel() // n
     elif x.dtype == torch.float32:
         if x.shape[-1] % 2:
             raise ValueError("interleaved input needs an even last dimension")
         n = x.shape[-1] // 2
-        xf = x
+        batch = x.numel() // (2 * n)
     else:
         raise TypeError("c2c takes complex64 or interleaved float32")
-    batch = x.numel() // (n * (1 if x.dtype == torch.complex64 else 2))
     out = torch.empty_like(x)
     if batch == 0:
         return out
-    of = torch.view_as_real(out) if x.dtype == torch.complex64 else out
     factor = norm_scale(n, sign, norm) if scale is None else scale
-    c2c_raw(xf, of, n, batch, sign, scale=None if factor == 1.0 else factor)
+    c2c_raw(x, out, n, batch, sign, scale=None if factor == 1.0 else factor)
     return out
 
 
@@ -145,7 +152,7 @@ def c2c_rows(x: torch.Tensor, sign: int = -1, out: torch.Tensor | None = None) -
     tab = table(_lib.KIND_C2C, n, x.device)
     work = workspace(_lib.KIND_C2C, n, batch, x.device) if n > 16384 else None
     rc = _lib.hip().bfly_c2c_rows(x.data_ptr(), idist, out.data_ptr(), odist, n, batch, sign, tab.data_ptr(),
-                                  work.data_ptr() if work is not None else None, _stream(x.device))
+                                  work.data_ptr() if work is not None else None, _stream(x))
     _lib.check(rc, f"bfly_c2c_rows(n={n}, batch={batch}, idist={idist}, odist={odist}, sign={sign})")
     return out
 
@@ -169,14 +176,14 @@ def table2d_cols(n1: int, device) -> torch.Tensor:
 
 def fft2_raw(x: torch.Tensor, out: torch.Tensor, n1: int, n2: int, batch: int, sign: int = -1,
              work: torch.Tensor | None = None) -> None:
-    """bfly_fft2d on interleaved float32 buffers [batch][n1][2 n2]."""
+    """bfly_fft2d on complex64 or interleaved float32 buffers of [batch][n1][n2] points."""
     lib = _lib.hip()
     if work is None:
         work = torch.empty(max(1, lib.bfly_fft2d_workspace_bytes(n1, n2, batch) // 4), dtype=torch.float32,
                            device=x.device)
     rc = lib.bfly_fft2d(x.data_ptr(), out.data_ptr(), n1, n2, batch, sign,
                         table(_lib.KIND_C2C, n2, x.device).data_ptr(), table2d_cols(n1, x.device).data_ptr(),
-                        work.data_ptr(), _stream(x.device))
+                        work.data_ptr(), _stream(x))
     _lib.check(rc, f"bfly_fft2d(n1={n1}, n2={n2}, batch={batch}, sign={sign})")
 
 
@@ -196,7 +203,7 @@ def fft_columns(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
     work = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device) if nbytes else None
     rc = lib.bfly_c2c_columns(x.data_ptr(), out.data_ptr(), n, ncols, batch, sign,
                               table2d_cols(n, x.device).data_ptr(), work.data_ptr() if work is not None else None,
-                              _stream(x.device))
+                              _stream(x))
     _lib.check(rc, f"bfly_c2c_columns(n={n}, ncols={ncols}, batch={batch}, sign={sign})")
     return out
 
@@ -213,7 +220,9 @@ def fft2(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
     out = torch.empty_like(x)
     if batch == 0:
         return out
-    fft2_raw(torch.view_as_real(x), torch.view_as_real(out), n1, n2, batch, sign)
+    if x.is_conj():
+        torch.view_as_real(x)  # raises: the memory holds the conjugate
+    fft2_raw(x, out, n1, n2, batch, sign)
     return out
 
 
@@ -222,7 +231,7 @@ def _real(kind: int, src: torch.Tensor, dst: torch.Tensor, n: int, batch: int, b
     tab = table(kind, n, src.device)
     rc = _lib.hip().bfly_real_ex(kind, src.data_ptr(), dst.data_ptr(), n, batch, bins, stride,
                                  _lib.VARIANT_AUTO, _lib.REAL_ADJOINT if adjoint else 0, tab.data_ptr(),
-                                 _stream(src.device))
+                                 _stream(src))
     _lib.check(rc, f"{what}(n={n}, batch={batch}, bins={bins}, adjoint={adjoint})")
 
 
@@ -303,14 +312,14 @@ def mode_mix(op: int, a: torch.Tensor, b: torch.Tensor, batch: int, c_in: int, c
         raise ValueError(f"unknown mode_mix op {op}")
     out = torch.empty(shape, dtype=torch.complex64, device=a.device)
     rc = _lib.hip().bfly_mode_mix(op, a.data_ptr(), b.data_ptr(), out.data_ptr(), batch, c_in, c_out, modes,
-                                  _stream(a.device))
+                                  _stream(a))
     _lib.check(rc, f"bfly_mode_mix(op={op}, batch={batch}, c_in={c_in}, c_out={c_out}, modes={modes})")
     return out
 
 
 def probe_copy(src: torch.Tensor, dst: torch.Tensor) -> None:
     rc = _lib.hip().bfly_probe_copy(src.data_ptr(), dst.data_ptr(), src.numel() * src.element_size(),
-                                    _stream(src.device))
+                                    _stream(src))
     _lib.check(rc, "bfly_probe_copy")
 
 
