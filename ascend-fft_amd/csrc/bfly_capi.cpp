@@ -310,8 +310,9 @@ static int c2c_checked(const float* in, float* out, uint32_t n, uint32_t batch, 
     if (int g = bfly_host::check_execute(BFLY_KIND_C2C, sign, in, out, n, batch, table, work, variant))
         return g;
     if (variant < BFLY_VARIANT_AUTO || variant > BFLY_VARIANT_LAST) return BFLY_ERR_SHAPE;
-    if (variant == BFLY_VARIANT_AUTO) variant = bfly_host::auto_kernel(n, batch);
+    // what a call needs and refuses follows the variant it names, whichever kernel runs
     const bool uses_work = bfly_host::needs_work(BFLY_KIND_C2C, n, batch, variant);
+    if (variant == BFLY_VARIANT_AUTO) variant = bfly_host::auto_kernel(n, batch);
     if (!bfly_host::disjoint(BFLY_KIND_C2C, in, out, uses_work ? work : nullptr, n, batch, 0, 0))
         return BFLY_ERR_SHAPE;
     return launched(bfly_kern::c2c(in, out, n, batch, sign, variant, table, work, S(stream), nullptr, scale));

@@ -621,11 +621,9 @@ __global__ __launch_bounds__(WG) void k_long_cols(
     // the first LDS exchange of the FFT orders the table writes before any read
     run_plan_lt<I1, T, DIR, LX_PAD>(v, lds + c * STRIDE, 0, t1s, t1s, t1s, t, std::make_index_sequence<2>{});
     float2* dst = ws + b * N + n2;
-    // The intermediate is read back by the row kernel right after: from
-    // 2^24 points per launch up it is written (and read) with ordinary,
-    // temporal accesses (65536 x 256: 98.5 -> 93.3 us, 32768 x 512: 94.9 ->
-    // 87.1), below that with the streaming hint (65536 x 64: 28.2 against
-    // 30.6 us temporal).  `temporal` is uniform.
+    // The intermediate is read back by the row kernel right after; `temporal`
+    // (uniform): written with ordinary accesses instead of the streaming hint
+    // (see launch_long_dir).
     auto store = [&](auto tmp) {
 #pragma unroll
         for (int m = 0; m < P / RL; m++)
@@ -746,8 +744,8 @@ __global__ __launch_bounds__(WG) void k_long_rows(
     const uint64_t b = blockIdx.x / GROUPS;
     const int k1_0 = (blockIdx.x % GROUPS) * C;
     constexpr uint64_t N = (uint64_t)N1 * N2;
-    // Stage the C contiguous rows through LDS (row-linear, coalesced); the
-    // intermediate's access hint follows k_long_cols (`temporal` is uniform).
+    // Stage the C contiguous rows through LDS (row-linear, coalesced);
+    // `temporal` (uniform) as in k_long_cols.
     const float2* src = ws + b * N + (uint64_t)k1_0 * N2;
     auto stage = [&](auto tmp) {
 #pragma unroll
@@ -991,7 +989,16 @@ hipError_t launch_long_dir(const float2* in, float2* out, float2* ws, const floa
     // measured slower in 512-thread workgroups.
     constexpr int C1w = 512 / PlanOf<I1>::T, C1 = bfly_plan::kBlock / PlanOf<I1>::T;
     constexpr int C2 = bfly_plan::kBlock / PlanOf<I2>::T;
-    const int temporal = (uint64_t)batch * N1 * N2 >= (1ull << 24) ? 1 : 0;
+    // Access hints of the intermediate, by what the launch moves.  While input,
+    // intermediate and output fit the last-level cache together, streaming
+    // stores are faster (65536 x 64: 28.3 against 29.1 us, x 32: 15.1 against
+    // 21; 32768 x 200: 42.5 against 43); beyond, ordinary ones (65536 x 72:
+    // 34.8 -> 31.8, x 128: 52.6 -> 49.8, x 192: 76.4 -> 67.8; 32768 x 300: 58.5
+    // -> 56.2).  Ordinary loads pay from 2^24 points only (65536 x 256: 89.3
+    // -> 88; x 128: 49.8 -> 49.3, x 72: 31.8 -> 33.6).
+    const uint64_t points = (uint64_t)batch * N1 * N2;
+    const int temporal = points > (N1 * N2 == 65536 ? 1ull << 22 : 1ull << 23) ? 1 : 0;
+    const int temporal_rows = points >= (1ull << 24) ? 1 : 0;
     static bfly_kern::ResidentCache rc;
     const int fit = bfly_kern::resident(rc, reinterpret_cast<const void*>(&k_long_cols<I1, N2, DIR, 512>), 512);
     const uint64_t units = (uint64_t)batch * (N2 / C1w);
@@ -1016,7 +1023,7 @@ hipError_t launch_long_dir(const float2* in, float2* out, float2* ws, const floa
             if (e != hipSuccess) return e;
             if (mid && (e = hipEventRecord(mid, s)) != hipSuccess) return e;
             hipLaunchKernelGGL((k_long_rows<I2, N1, DIR>), dim3(batch * (N1 / C2)), dim3(bfly_plan::kBlock),
-                               0, s, ws, out, tw2, scale, odist, temporal);
+                               0, s, ws, out, tw2, scale, odist, temporal_rows);
             return hipGetLastError();
         }
     }
@@ -1030,7 +1037,7 @@ hipError_t launch_long_dir(const float2* in, float2* out, float2* ws, const floa
     if (e != hipSuccess) return e;
     if (mid && (e = hipEventRecord(mid, s)) != hipSuccess) return e;
     hipLaunchKernelGGL((k_long_rows<I2, N1, DIR>), dim3(batch * (N1 / C2)), dim3(bfly_plan::kBlock),
-                       0, s, ws, out, tw2, scale, odist, temporal);
+                       0, s, ws, out, tw2, scale, odist, temporal_rows);
     return hipGetLastError();
 }
 

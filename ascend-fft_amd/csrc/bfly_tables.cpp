@@ -287,11 +287,12 @@ int auto_variant(uint32_t n, uint32_t batch) {
 // One transform per workgroup with 32 points per thread (bfly_wide.hip),
 // measured against auto_variant's kernel: 8192 b=64 9.0 against 9.0 us, b=256
 // 10.7 against 11.5, b=2048 49.6 against 54.4; 16384 b=256 17.6 against 18.9,
-// b=1000 56.3 against 59.4 (below 256 the four-step chain's wider grid wins,
-// b=128: 14.1 against 15.5); 32768 b=128 26.0 against 25.5 for the four-step
+// b=1000 56.3 against 59.4, b=255 17.5 against 26.8 for the four-step chain
+// and b=160 15.8 both (below, the chain's wider grid wins, b=128: 14.1 against
+// 15.3); 32768 b=128 26.0 against 25.5 for the four-step
 // chain, b=144 27.0 against 32.1, b=256 32.0 against 51.3.
 int auto_kernel(uint32_t n, uint32_t batch) {
-    if ((n == 8192 && batch >= 128) || (n == 16384 && batch >= 256) || (n == 32768 && batch > 128))
+    if ((n == 8192 && batch >= 128) || (n == 16384 && batch >= 160) || (n == 32768 && batch > 128))
         return kVariantWide;
     return auto_variant(n, batch);
 }

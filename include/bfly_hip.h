@@ -205,7 +205,7 @@ BFLY_API int bfly_c2c_scaled(const float* in, float* out, uint32_t n, uint32_t b
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): same
  * arguments minus `work`, same kernels, same results bit for bit.  No
  * counterpart in the reference.  The four-step chain's intermediate (the
- * only scratch a C2C uses: n > 16384, and 16384 with batch < 256) lives in a
+ * only scratch a C2C uses: n > 16384, and 16384 with batch < 160) lives in a
  * static device array of BFLY_NOALLOC_SCRATCH_BYTES per GPU, held until the
  * process ends; a shape whose intermediate (8 n batch bytes) does not fit
  * returns BFLY_ERR_SCRATCH (at 64 MiB: n * batch <= 8388608, e.g. 65536 x
@@ -309,9 +309,9 @@ BFLY_API int bfly_c2c_traced(const float* in, float* out, uint32_t n, uint32_t b
  * STREAM_LT run one workgroup per transform (one-shot / streaming) and the
  * other ids the one-shot form; above 16384 every id runs four-step.  AUTO
  * runs a kernel of its own, one transform per workgroup of n/32 threads, at
- * 8192 from 128 transforms, at 16384 from 256 and at 32768 above 128 (there
- * the workspace is asked for all the same, and bfly_c2c_launches and
- * bfly_c2c_traced report and time the four-step chain). */
+ * 8192 from 128 transforms, at 16384 from 160 and at 32768 above 128 (at
+ * 16384 below 256 and at 32768 the workspace is asked for all the same, and
+ * bfly_c2c_launches and bfly_c2c_traced report and time the four-step chain). */
 #define BFLY_VARIANT_AUTO 0
 #define BFLY_VARIANT_PLAIN 1
 #define BFLY_VARIANT_STREAM 2

@@ -16,8 +16,10 @@ REL_L2 = 2e-6
 
 # below, at and above the batch from which AUTO picks the kernel; more than one
 # round of resident workgroups
-CASES = [(8192, 127), (8192, 128), (8192, 1301), (16384, 255), (16384, 256), (16384, 601), (32768, 128),
-         (32768, 129), (32768, 301)]
+CASES = [(8192, 127), (8192, 128), (8192, 1301), (16384, 159), (16384, 160), (16384, 255), (16384, 256),
+         (16384, 601), (32768, 128), (32768, 129), (32768, 301),
+         # the two-kernel chain on both sides of the size from which its intermediate's stores are ordinary ones
+         (65536, 64), (65536, 65)]
 
 
 def _rows(t, pick, n):
