@@ -8,8 +8,8 @@
 // through the batch, so a group may span two items and no lane idles where
 // the columns per item are few or no multiple of C.  Two kernels:
 //
-//   k_cols       16 points per thread, up to 256-point columns (and few
-//                512-point ones): 256-thread workgroups, C >= 16;
+//   k_cols       16 points per thread, up to 256-point columns (and 512- and
+//                1024-point ones in few groups): C >= 16;
 //   k_cols_wide  32 points per thread (bfly_wide.hpp), 512 to 4096 points in
 //                256 / 512 / 1024-thread workgroups (launch_wide).
 //
@@ -47,8 +47,8 @@ struct ColView {
     uint32_t in_rstride, out_rstride;
     uint32_t ncols, mats, total;
     uint32_t col_div;  // twiddle pass: q = column / col_div
-    int temporal;      // see line_aligned
-    uint32_t win;      // units per XCD window (set by the launcher)
+    int temporal;      // bit 0 / 1: loads / stores without the streaming hint (line_aligned)
+    uint32_t win;      // units per XCD window; 0: the launcher's choice
 };
 
 // Rows that start on 128-byte lines: a run of 16 or more columns then covers
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
                     active ? ld_io<decltype(nt)::value>(&src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))])
                            : make_float2(0.f, 0.f);
     };
-    if (cv.temporal) load(std::false_type{});
+    if (cv.temporal & 1) load(std::false_type{});
     else load(std::true_type{});
     tabs.park(ltw, tid);
     if constexpr (TW)
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
                 st_io<decltype(nt)::value>(&dst[(uint64_t)cv.out_rstride * k], x);
             }
     };
-    if (cv.temporal) store(std::false_type{});
+    if (cv.temporal & 2) store(std::false_type{});
     else store(std::true_type{});
 }
 
@@ -278,27 +278,44 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, con
     return hipGetLastError();
 }
 
-// Picks the wide kernel's workgroup: the largest that still gives every CU
-// one.  A larger one takes longer runs (256 bytes at 1024 points and 1024 threads)
-// and, at 1024 threads, the whole LDS of a CU, which pays where a run is
-// whole lines (1024 x 1024 x 16: 48.7 us against 55.7 at 512 threads; 2048 x
-// 1024 x 8: 55.0 against 75.9) or, at 4096 points, too short anyway (4096 x
-// 1024 x 4: 69.3 against 85.5; 4096 x 333 x 4: 34.5 against 39.7); other rows
-// run best at 512 threads, two workgroups to a CU (2048 x 999 x 6: 55.1
-// against 62.6).  Few columns: 256 threads (1024 x 64 x 4: 6.9 us against
-// 10.4 at 512 threads; 2048 x 100 x 8: 11.5 against 13.9).
+// Picks the wide kernel's workgroup.  256, 512 and 1024 threads keep the same
+// number of columns resident (four, two and one workgroup to a CU), so the
+// smallest that still gives every CU at most one workgroup is the fastest:
+// with a few more, some CUs run two while the others wait (whole-line rows,
+// the smaller -> the larger workgroup: 2-D 2048 x 256 x 12 53.0 -> 45.0 us,
+// 1024 x 1024 x 6 45.4 -> 41.3, 4096 x 256 x 6 67.1 -> 50.0; one size too large:
+// 1024 x 1024 x 2 19.5 -> 22.3).  Beyond one to a CU, whole-line rows take
+// 1024 threads: longer runs (256 bytes at 1024 points; 1024 x 1024 x 16: 48.7
+// us against 55.7 at 512, 2048 x 1024 x 8: 55.0 against 75.9).  The lines below
+// are where the measurements leave this rule.
 template <int L>
 hipError_t launch_wide(const float2* in, float2* out, const float2* tc, const float2* wab, uint32_t ncols,
                        uint32_t total, bool aligned, bool rows_behind, int sign, hipStream_t s) {
-    constexpr uint32_t kCus = 256;
-    // (right behind the 2-D transform's row pass, narrow matrices run better
-    // at 512 threads: 2-D 1024 x 128 x 128 90.4 us against 95.1, where the
-    // column pass by itself takes 61.1 against 51.8)
-    if constexpr (L >= 1024)
-        if ((aligned || L == 4096) && !(L == 1024 && rows_behind && ncols < 256) && total >= kCus * (32768u / L))
+    constexpr uint32_t kOne = 256 * (16384 / L);  // columns of one 512-thread workgroup per CU
+    if constexpr (L == 512) {
+        // 256 threads: whole-line rows of few columns (512 x 256 x 80 73.0 us
+        // against 65.5 at 512 threads, x 128 105 against 99; 512 columns 63.5
+        // against 66.5), other rows up to three quarters of the resident
+        // columns (512 x 999 x 12 20.1 against 18.0, x 16 25.3 against 26.8)
+        if (aligned ? ncols <= 256 : total <= 12288)
+            return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
+    } else if constexpr (L == 4096) {
+        if (total > kOne) return launch_cols_wide<L, 1024>(in, out, tc, wab, ncols, total, aligned, sign, s);
+    } else if (aligned) {
+        // narrow matrices, behind the 2-D transform's row pass or in less than
+        // a round, run better at 512 threads (2-D 1024 x 128 x 128 90.4 us
+        // against 95.1, where the column pass by itself takes 61.1 against
+        // 51.8; 1024 x 128 x 48 39.9 against 41.5)
+        const bool narrow = ncols < 256 && (total < 2 * kOne || (L == 1024 && rows_behind));
+        if (total > kOne && !narrow)
             return launch_cols_wide<L, 1024>(in, out, tc, wab, ncols, total, aligned, sign, s);
-    // (2048 points: from half that, 2-D 2048 x 256 x 4 22.5 us against 26.8)
-    if (L == 4096 || total >= kCus * (16384u / L) / (L == 2048 && aligned ? 2 : 1))
+    } else if (L == 1024 && total <= 6144) {
+        // (1024 x 999 x 6 21.4 us against 22.3 at 512 threads, x 7 32.6 against 26.6)
+        return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
+    }
+    // (2048 points: 512 threads from half a round, 2-D 2048 x 256 x 4 23.2 us
+    // against 24.0, x 2 22.2 against 20.2)
+    if (L == 4096 || total >= kOne / (L == 2048 && aligned ? 2 : 1))
         return launch_cols_wide<L, 512>(in, out, tc, wab, ncols, total, aligned, sign, s);
     if constexpr (L < 4096) return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
     return hipErrorInvalidValue;
@@ -310,8 +327,10 @@ hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const fl
     constexpr uint32_t C = WG / PlanOf<I>::T;
     const uint32_t blocks = (uint32_t)(((uint64_t)cv.total + C - 1) / C);
     // whole-line rows in a round of workgroups or less: as dealt (the split's
-    // first pass at 4096 x 64 x 4 5.4 us against 6.6)
-    cv.win = cv.temporal || blocks >= 1024 ? kColWindow : 1;
+    // first pass at 4096 x 64 x 4 5.4 us against 6.6); 64 and 128 points
+    // always (128 x 2048 x 64 46.2 us against 59.0 in windows, other widths equal)
+    constexpr int L = PlanOf<I>::N;
+    if (!cv.win) cv.win = blocks >= 1024 && L != 64 && L != 128 ? kColWindow : 1;
     if (sign < 0)
         hipLaunchKernelGGL((k_cols<I, -1, TW, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
     else
@@ -334,9 +353,12 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
     const uint32_t F = (uint32_t)total;
     const bool al = line_aligned(in, out, ncols);
     constexpr auto idx = bfly_plan::plan_index;
-    // (16 and 32 points: runs of 2 and 1 KiB are mostly whole lines however
-    // the rows start: 16 x 1000 x 700 32.6 us with the hint, 34.7 without)
-    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, al || n1 <= 32 ? 0 : 1, 1};
+    // (16 and 32 points, whose runs of 2 and 1 KiB are mostly whole lines
+    // however the rows start, past what the last-level cache holds: 16 x 1000
+    // x 700 32.6 us with the hint, 34.7 without; 16 x 1000 x 400 20.4 against
+    // 17.2, 32 x 167 x 500 11.6 against 9.3)
+    const bool hint = al || (n1 <= 32 && item * batch > (1ull << 23));
+    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, hint ? 0 : 3, al ? 0 : kColWindow};
     const float2* t1 = tc + L.p_table;
     switch (n1) {
         case 16: return launch_cols<idx(16), false>(i2, o2, t1, nullptr, cv, sign, s);
@@ -350,7 +372,14 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
             // 64 x 128 11.6 against 12.7 (512 x 64 x 256: 26.4 against 23.1)
             if (al && F < 12288) return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, sign, s);
             return launch_wide<512>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
-        case 1024: return launch_wide<1024>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
+        case 1024:
+            // whole-line rows, more columns than 256-thread workgroups take in
+            // one per CU and fewer than 512-thread ones: 2-D 1024 x 1024 x 3
+            // 24.2 us against 29.6 and 23.9, 1024 x 128 x 24 23.5 against 29.1
+            // and 26.1, 1024 x 64 x 40 23.2 against 24.6 and 27.0
+            if (al && F > 2048 && F < 4096)
+                return launch_cols<idx(1024), false, 1024>(i2, o2, t1, nullptr, cv, sign, s);
+            return launch_wide<1024>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
         case 2048: return launch_wide<2048>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
         default: break;
     }
@@ -359,10 +388,16 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
     // P-point pass with the twiddle: in -> ws; Q-point pass with the row map: ws -> out
     float2* ws = reinterpret_cast<float2*>(work);
     const uint32_t qn = L.q * ncols;
-    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, line_aligned(in, ws, qn) ? 0 : 1, 1};
+    const bool whole = line_aligned(in, ws, qn);
+    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, whole ? 0 : 3, whole ? 0 : kColWindow};
     hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, wab, a, sign, s);
     if (e != hipSuccess) return e;
-    const ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, L.p, qn * batch, 1, line_aligned(ws, out, ncols) ? 0 : 1, 1};
+    // (with the hint from 16 columns however the rows start: read without it,
+    // the lines of the workspace slow the next call's first pass, as above:
+    // 4096 x 60 x 7 14.4 us against 18.5; 4096 x 3 x 214 25.7 against 21.7)
+    const bool own = line_aligned(ws, out, ncols);
+    const ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, L.p, qn * batch, 1, own || ncols >= 16 ? 0 : 3,
+                    own ? 0 : kColWindow};
     return launch_cols<idx(64), false>(ws, o2, tc + L.q_table, nullptr, b, sign, s);
 }
 

@@ -19,7 +19,12 @@ REL_L2 = 1e-6
 # from 256 groups of 16384 points on 512 threads, of 32768 points 1024
 SHAPES = [(512, 1, 5), (512, 33, 3), (512, 31, 300), (512, 64, 200), (1024, 15, 3), (1024, 17, 250), (1024, 48, 100),
           (1024, 64, 130), (2048, 3, 5), (2048, 30, 40), (2048, 7, 320), (2048, 16, 257), (4096, 1, 3),
-          (4096, 11, 100), (4096, 9, 230), (4096, 16, 129)]
+          (4096, 11, 100), (4096, 9, 230), (4096, 16, 129),
+          # between one 256-, 512- and 1024-thread workgroup per CU, and the two-pass split's ragged rows
+          (1024, 256, 10), (1024, 256, 21), (2048, 256, 9), (4096, 64, 17), (512, 256, 50), (1024, 333, 17),
+          (4096, 20, 50),
+          # shorter columns (16 points per thread): windows, and 16 points on both sides of 2^23
+          (16, 167, 50), (16, 999, 530), (32, 100, 90), (128, 2048, 17), (256, 64, 300)]
 
 
 def _columns(x, sign):
