@@ -47,8 +47,10 @@ struct ColView {
     uint32_t in_rstride, out_rstride;
     uint32_t ncols, mats, total;
     uint32_t col_div;  // twiddle pass: q = column / col_div
-    int temporal;      // bit 0 / 1: loads / stores without the streaming hint (line_aligned)
-    uint32_t win;      // units per XCD window; 0: the launcher's choice
+    int temporal;      // without the streaming hint (line_aligned)
+    uint32_t win;      // log2 of the units per XCD window (kAutoWindow: the launcher's choice)
+    Divider unit;      // set by the launcher: by the groups per matrix if whole, else by its columns
+    Divider mat;       // set by the launcher: by mats
 };
 
 // Rows that start on 128-byte lines: a run of 16 or more columns then covers
@@ -64,7 +66,8 @@ bool line_aligned(const void* in, const void* out, uint32_t ncols) {
 // 8 / 16 / 64 of the 16-point kernel: 512 x 1001 x 24 66.6 / 58.3 / 53.1 /
 // 50.8 / 50.4 / 54.3 us, 256 x 1024 x 64 55.3 / 55.1 / 54.4 / 51.3 / 48.9 us
 // (1 .. 16), 64 x 1001 x 200 53.5 / 49.2 / 46.0 / 44.6 / 42.6 / 42.6.
-constexpr uint32_t kColWindow = 16;
+constexpr uint32_t kColWindow = 4;  // log2
+constexpr uint32_t kAutoWindow = ~0u;
 
 // 4096-point columns from which one pass is used (4096 x 64 x 16, 1024 of
 // them: 18.5 us against 27.9 in two passes, 2-D 4096 x 256 x 4 41.0 against
@@ -74,7 +77,9 @@ constexpr uint32_t kOnePassCols = 1024;
 // One column group per workgroup: C = WG / T adjacent columns, 16 points per
 // thread.  Bound by HBM (run lengths of C columns); columns up to 256 points,
 // and 512-point ones in few groups (column_pass).
-template <int I, int DIR, bool TW, int WG = bfly_plan::kBlock>
+// HINT: streaming accesses (a template argument: both forms in one kernel cost
+// a launch 0.1 us more, 256 x 256 x 8 5.04 -> 4.95).
+template <int I, int DIR, bool TW, int WG, bool HINT>
 __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ wab,
                                               ColView cv) {
@@ -95,35 +100,25 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
     C2cLdsTwFetch<I, WG> tabs;
     tabs.fetch(tw, tw + bfly_plan::stage_twiddle_len(I), tid);
     const int c = tid % C, t = tid / C;
-    const uint32_t blk = xcd_window(blockIdx.x, gridDim.x, cv.win), f = blk * C + c;
+    const uint32_t blk = xcd_window_log2(blockIdx.x, gridDim.x, cv.win), f = blk * C + c;
     const bool active = f < cv.total;
     uint32_t mi, col;  // matrix and column of this lane
     if (cv.ncols % C == 0) {  // whole groups: one division per workgroup
-        const uint32_t groups = cv.ncols / C;
-        mi = blk / groups;
-        col = (blk - mi * groups) * C + c;
+        mi = cv.unit.divide(blk, &col);
+        col = col * C + c;
     } else {
-        mi = f / cv.ncols;
-        col = f - mi * cv.ncols;
+        mi = cv.unit.divide(f, &col);
     }
     uint32_t b = mi, m = 0;
-    if (cv.mats > 1) {
-        b = mi / cv.mats;
-        m = mi - b * cv.mats;
-    }
+    if (cv.mats > 1) b = cv.mat.divide(mi, &m);
     const float2* src = in + b * cv.item + m * cv.in_mstride + col;
     float2 v[P];
-    auto load = [&](auto nt) {
 #pragma unroll
-        for (int mm = 0; mm < P / R0; mm++)
+    for (int mm = 0; mm < P / R0; mm++)
 #pragma unroll
-            for (int r = 0; r < R0; r++)
-                v[mm * R0 + r] =
-                    active ? ld_io<decltype(nt)::value>(&src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))])
-                           : make_float2(0.f, 0.f);
-    };
-    if (cv.temporal & 1) load(std::false_type{});
-    else load(std::true_type{});
+        for (int r = 0; r < R0; r++)
+            v[mm * R0 + r] = active ? ld_io<HINT>(&src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))])
+                                    : make_float2(0.f, 0.f);
     tabs.park(ltw, tid);
     if constexpr (TW)
         for (int i = tid; i < 128; i += WG) wt[i] = wab[i];
@@ -133,23 +128,19 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
     if (!active) return;
     float2* dst = out + b * cv.item + m * cv.out_mstride + col;
     const uint32_t q = TW ? col / cv.col_div : 0u;
-    auto store = [&](auto nt) {
 #pragma unroll
-        for (int mm = 0; mm < P / RL; mm++)
+    for (int mm = 0; mm < P / RL; mm++)
 #pragma unroll
-            for (int r = 0; r < RL; r++) {
-                const int k = t + mm * T + r * (L / RL);
-                float2 x = v[mm * RL + r];
-                if constexpr (TW) {
-                    const uint32_t e = q * (uint32_t)k;  // < n1 <= 4096
-                    const float2 a = wt[e & 63], w = wt[64 + (e >> 6)];
-                    x = cmul_tw<DIR>(x, make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x));
-                }
-                st_io<decltype(nt)::value>(&dst[(uint64_t)cv.out_rstride * k], x);
+        for (int r = 0; r < RL; r++) {
+            const int k = t + mm * T + r * (L / RL);
+            float2 x = v[mm * RL + r];
+            if constexpr (TW) {
+                const uint32_t e = q * (uint32_t)k;  // < n1 <= 4096
+                const float2 a = wt[e & 63], w = wt[64 + (e >> 6)];
+                x = cmul_tw<DIR>(x, make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x));
             }
-    };
-    if (cv.temporal & 2) store(std::false_type{});
-    else store(std::true_type{});
+            st_io<HINT>(&dst[(uint64_t)cv.out_rstride * k], x);
+        }
 }
 
 // Plans of the wide column kernel: the second pass's twiddles come from its
@@ -194,7 +185,7 @@ __device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, const 
 template <int L, int DIR, int WG>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_cols_wide(
     const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tc,
-    const float2* __restrict__ wab, uint32_t ncols, uint32_t total, int stream_in,
+    const float2* __restrict__ wab, uint32_t ncols, Divider cols, uint32_t total, int stream_in,
     int stream_out, uint32_t win) {
     using P = ColPlan<L>;
     constexpr int T = L / kWide, C = WG / T, LO = 64, HI = L / LO;
@@ -209,9 +200,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     const int c = tid % C;
     int t = tid / C;
     // columns are numbered through the batch (f = item * ncols + column)
-    const uint32_t f = xcd_window(blockIdx.x, gridDim.x, win) * C + c;
+    const uint32_t f = xcd_window_log2(blockIdx.x, gridDim.x, win) * C + c;
     const uint32_t fr = f < total ? f : total - 1;  // past the end: reads the last column again
-    const uint64_t at = (uint64_t)(fr / ncols) * L * ncols + fr % ncols;
+    uint32_t col;
+    const uint32_t item = cols.divide(fr, &col);
+    const uint64_t at = (uint64_t)item * L * ncols + col;
     const float2* src = in + (at + (uint64_t)t * ncols);
     float2 v[kWide];
     auto load = [&](auto nt) {
@@ -268,12 +261,13 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, con
     // 26.9 against 29.1).
     const int in_hint = aligned;
     const int out_hint = aligned && (L == 512 || (L == 1024 && (WG < 1024 || blocks >= 512)) || (L == 2048 && WG == 512));
-    const uint32_t win = !aligned ? 32 : WG == 1024 ? (L == 1024 && ncols <= 256 ? 64 : 32) : WG == 512 && L < 2048 ? 32 : 4;
+    // (log2 of the window)
+    const uint32_t win = !aligned ? 5 : WG == 1024 ? (L == 1024 && ncols <= 256 ? 6 : 5) : WG == 512 && L < 2048 ? 5 : 2;
     if (sign < 0)
-        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, total,
+        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, Divider(ncols), total,
                            in_hint, out_hint, win);
     else
-        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, total,
+        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, Divider(ncols), total,
                            in_hint, out_hint, win);
     return hipGetLastError();
 }
@@ -330,11 +324,14 @@ hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const fl
     // first pass at 4096 x 64 x 4 5.4 us against 6.6); 64 and 128 points
     // always (128 x 2048 x 64 46.2 us against 59.0 in windows, other widths equal)
     constexpr int L = PlanOf<I>::N;
-    if (!cv.win) cv.win = blocks >= 1024 && L != 64 && L != 128 ? kColWindow : 1;
-    if (sign < 0)
-        hipLaunchKernelGGL((k_cols<I, -1, TW, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
-    else
-        hipLaunchKernelGGL((k_cols<I, 1, TW, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+    if (cv.win == kAutoWindow) cv.win = blocks >= 1024 && L != 64 && L != 128 ? kColWindow : 0;
+    cv.unit = Divider(cv.ncols % C == 0 ? cv.ncols / C : cv.ncols);
+    cv.mat = Divider(cv.mats);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+    };
+    if (cv.temporal) sign < 0 ? go(&k_cols<I, -1, TW, WG, false>) : go(&k_cols<I, 1, TW, WG, false>);
+    else sign < 0 ? go(&k_cols<I, -1, TW, WG, true>) : go(&k_cols<I, 1, TW, WG, true>);
     return hipGetLastError();
 }
 
@@ -358,7 +355,7 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
     // x 700 32.6 us with the hint, 34.7 without; 16 x 1000 x 400 20.4 against
     // 17.2, 32 x 167 x 500 11.6 against 9.3)
     const bool hint = al || (n1 <= 32 && item * batch > (1ull << 23));
-    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, hint ? 0 : 3, al ? 0 : kColWindow};
+    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, hint ? 0 : 1, al ? kAutoWindow : kColWindow, {}, {}};
     const float2* t1 = tc + L.p_table;
     switch (n1) {
         case 16: return launch_cols<idx(16), false>(i2, o2, t1, nullptr, cv, sign, s);
@@ -389,15 +386,15 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
     float2* ws = reinterpret_cast<float2*>(work);
     const uint32_t qn = L.q * ncols;
     const bool whole = line_aligned(in, ws, qn);
-    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, whole ? 0 : 3, whole ? 0 : kColWindow};
+    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, whole ? 0 : 1, whole ? kAutoWindow : kColWindow, {}, {}};
     hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, wab, a, sign, s);
     if (e != hipSuccess) return e;
     // (with the hint from 16 columns however the rows start: read without it,
     // the lines of the workspace slow the next call's first pass, as above:
     // 4096 x 60 x 7 14.4 us against 18.5; 4096 x 3 x 214 25.7 against 21.7)
     const bool own = line_aligned(ws, out, ncols);
-    const ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, L.p, qn * batch, 1, own || ncols >= 16 ? 0 : 3,
-                    own ? 0 : kColWindow};
+    const ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, L.p, qn * batch, 1, own || ncols >= 16 ? 0 : 1,
+                    own ? kAutoWindow : kColWindow, {}, {}};
     return launch_cols<idx(64), false>(ws, o2, tc + L.q_table, nullptr, b, sign, s);
 }
 
