@@ -64,6 +64,15 @@ def _check_device(t: torch.Tensor, name: str) -> None:
         raise ValueError(f"{name} must be contiguous")
 
 
+def plain(t: torch.Tensor) -> torch.Tensor:
+    """`t` with its memory holding its values: torch conjugates and negates
+    lazily, as a bit of the tensor, and a kernel reads the memory.  (contiguous()
+    keeps the bit of a tensor that is contiguous already.)"""
+    if t.is_conj():
+        t = t.resolve_conj()
+    return t.resolve_neg() if t.is_neg() else t
+
+
 def c2c_raw(x: torch.Tensor, out: torch.Tensor, n: int, batch: int, sign: int = -1,
             work: torch.Tensor | None = None, scale: float | None = None) -> None:
     """bfly_c2c on complex64 or interleaved float32 buffers (no allocation
@@ -123,7 +132,7 @@ def c2c(x: torch.Tensor, sign: int = -1, norm: str | None = None, *, scale: floa
     if batch == 0:
         return out
     factor = norm_scale(n, sign, norm) if scale is None else scale
-    c2c_raw(x, out, n, batch, sign, scale=None if factor == 1.0 else factor)
+    c2c_raw(plain(x), out, n, batch, sign, scale=None if factor == 1.0 else factor)
     return out
 
 
@@ -144,6 +153,9 @@ def c2c_rows(x: torch.Tensor, sign: int = -1, out: torch.Tensor | None = None) -
         raise ValueError("out must be a complex64 [batch][n] tensor on the input's device")
     if batch == 0:
         return out
+    if out.is_conj() or out.is_neg():
+        raise RuntimeError("out is a lazily conjugated or negated view: what is written to its memory reads otherwise")
+    x = plain(x)
     for t, name in ((x, "x"), (out, "out")):
         if t.stride(1) != 1 or (batch > 1 and t.stride(0) < n):
             raise ValueError(f"{name} rows must be unit-stride and at least n apart")
@@ -199,6 +211,7 @@ def fft_columns(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
     if batch == 0:
         return out
     lib = _lib.hip()
+    x = plain(x)
     nbytes = lib.bfly_c2c_columns_workspace_bytes(n, ncols, batch)
     work = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device) if nbytes else None
     rc = lib.bfly_c2c_columns(x.data_ptr(), out.data_ptr(), n, ncols, batch, sign,
@@ -222,12 +235,13 @@ def fft2(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
         return out
     if x.is_conj():
         torch.view_as_real(x)  # raises: the memory holds the conjugate
-    fft2_raw(x, out, n1, n2, batch, sign)
+    fft2_raw(plain(x), out, n1, n2, batch, sign)
     return out
 
 
 def _real(kind: int, src: torch.Tensor, dst: torch.Tensor, n: int, batch: int, bins: int, stride: int,
           adjoint: bool, what: str) -> None:
+    src = plain(src)
     tab = table(kind, n, src.device)
     rc = _lib.hip().bfly_real_ex(kind, src.data_ptr(), dst.data_ptr(), n, batch, bins, stride,
                                  _lib.VARIANT_AUTO, _lib.REAL_ADJOINT if adjoint else 0, tab.data_ptr(),
@@ -311,6 +325,7 @@ def mode_mix(op: int, a: torch.Tensor, b: torch.Tensor, batch: int, c_in: int, c
     if shape is None:
         raise ValueError(f"unknown mode_mix op {op}")
     out = torch.empty(shape, dtype=torch.complex64, device=a.device)
+    a, b = plain(a), plain(b)
     rc = _lib.hip().bfly_mode_mix(op, a.data_ptr(), b.data_ptr(), out.data_ptr(), batch, c_in, c_out, modes,
                                   _stream(a))
     _lib.check(rc, f"bfly_mode_mix(op={op}, batch={batch}, c_in={c_in}, c_out={c_out}, modes={modes})")
