@@ -144,7 +144,7 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
 }
 
 // Plans of the wide column kernel: the second pass's twiddles come from its
-// own LDS table, the third pass's from the two-level tables.
+// own LDS table, the third pass's from wide_table.
 template <int L>
 struct ColPlan;
 template <> struct ColPlan<512> { static constexpr int R0 = 32, R1 = 16, R2 = 1; };
@@ -152,9 +152,10 @@ template <> struct ColPlan<1024> { static constexpr int R0 = 32, R1 = 32, R2 = 1
 template <> struct ColPlan<2048> { static constexpr int R0 = 16, R1 = 4, R2 = 32; };
 template <> struct ColPlan<4096> { static constexpr int R0 = 16, R1 = 8, R2 = 32; };
 
-// W_L^m, m < L, from the column table of L.
+// W_L^m from the column table of L; 2048 and 4096 points: m a multiple of 32
+// (the 4096-point table holds W_4096^j only for j < 64 and multiples of 64).
 template <int L>
-__device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, const float2* __restrict__ wab, int m) {
+__device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, int m) {
     if constexpr (L == 512) {  // last pass of 16 16 2: W^k at [256 + 2 k + 1], k < 256
         const float2 w = tc[256 + 2 * (m & 255) + 1];
         return m & 256 ? make_float2(-w.x, -w.y) : w;
@@ -162,12 +163,12 @@ __device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, const 
         const float2 w = tc[256 + 4 * (m & 255) + 1];
         const int q = m >> 8;
         return q == 0 ? w : q == 1 ? make_float2(w.y, -w.x) : q == 2 ? make_float2(-w.x, -w.y) : make_float2(-w.y, w.x);
-    } else if constexpr (L == 2048) {  // 16 16 8: W^{4 k} at [256 + 8 k + 4], k < 256; here m is a multiple of 32
+    } else if constexpr (L == 2048) {  // 16 16 8: W^{4 k} at [256 + 8 k + 4], k < 256
         const float2 w = tc[256 + 8 * ((m & 1023) / 4) + 4];
         return m & 1024 ? make_float2(-w.x, -w.y) : w;
     } else {
-        const float2 a = wab[m & 63], b = wab[64 + (m >> 6)];
-        return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+        const Wide64 w = root64(m, L);
+        return make_float2((float)w.x, (float)w.y);
     }
 }
 
@@ -184,18 +185,18 @@ __device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, const 
 // 1001 x 12 98.4 -> 52.9, 2048 x 999 x 6 120 -> 54, 4096 x 333 x 9 91.5 -> 73.
 template <int L, int DIR, int WG>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_cols_wide(
-    const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tc,
-    const float2* __restrict__ wab, uint32_t ncols, Divider cols, uint32_t total, int stream_in,
-    int stream_out, uint32_t win) {
+    const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tc, uint32_t ncols,
+    Divider cols, uint32_t total, int stream_in, int stream_out, uint32_t win) {
     using P = ColPlan<L>;
-    constexpr int T = L / kWide, C = WG / T, LO = 64, HI = L / LO;
+    constexpr int T = L / kWide, C = WG / T;
     // columns lie 32 / C banks apart (mod 64), so that the C columns and the
     // 32 / C consecutive points of a half-wave's access hit 32 banks
     constexpr int SH = C >= 32 ? 1 : 32 / C;
     constexpr int STRIDE = lds_len(L) + (SH - lds_len(L) % 64 + 64) % 64;
     constexpr int T1 = P::R0 * P::R1;
     __shared__ float lds[C * STRIDE];
-    __shared__ float2 tab[T1 + (P::R2 > 1 ? LO + HI : 0)];
+    __shared__ float2 t1[T1];
+    __shared__ Wide64 tab[P::R2 > 1 ? kWideTab<L> : 1];
     const int tid = threadIdx.x;
     const int c = tid % C;
     int t = tid / C;
@@ -218,16 +219,12 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     else load(std::false_type{});
     // the tables, behind the columns' loads (ahead of them they held the
     // loads back: 2048 x 1024 x 4 27.5 -> 30.3 us)
-    const float2 *t1 = tab, *tlo = tab + T1, *thi = tlo + LO;
-    for (int i = tid; i < T1; i += WG) tab[i] = col_root<L>(tc, wab, (i / P::R0) * (i % P::R0) * (L / T1));
+    for (int i = tid; i < T1; i += WG) t1[i] = col_root<L>(tc, (i / P::R0) * (i % P::R0) * (L / T1));
     if constexpr (P::R2 > 1) {
-        const float2* ab = L == 4096 ? wab : tc + bfly_plan::stage_twiddle_len(bfly_plan::plan_index(L));
-        for (int i = tid; i < LO + HI; i += WG) tab[T1 + i] = ab[i];
-    }
-    if constexpr (P::R2 > 1) {
-        stockham_wide<L, T, DIR, LO, P::R0, 1, P::R0, P::R1, P::R2>(v, lds + c * STRIDE, tlo, thi, t1, t);
+        wide_table<L>(tab, tid);
+        stockham_wide<L, T, DIR, P::R0, 1, P::R0, P::R1, P::R2>(v, lds + c * STRIDE, tab, t1, t);
     } else {
-        stockham_wide<L, T, DIR, LO, P::R0, 1, P::R0, P::R1>(v, lds + c * STRIDE, tlo, thi, t1, t);
+        stockham_wide<L, T, DIR, P::R0, 1, P::R0, P::R1>(v, lds + c * STRIDE, tab, t1, t);
     }
     if (f >= total) return;
     constexpr int RL = P::R2 > 1 ? P::R2 : P::R1;
@@ -245,8 +242,8 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 }
 
 template <int L, int WG>
-hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, const float2* wab, uint32_t ncols,
-                            uint32_t total, bool aligned, int sign, hipStream_t s) {
+hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, uint32_t ncols, uint32_t total,
+                            bool aligned, int sign, hipStream_t s) {
     constexpr uint32_t C = WG / (L / kWide);
     const uint32_t blocks = (uint32_t)(((uint64_t)total + C - 1) / C);
     // Access hints and windows (kColWindow: why windows; line_aligned: why
@@ -264,11 +261,11 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, con
     // (log2 of the window)
     const uint32_t win = !aligned ? 5 : WG == 1024 ? (L == 1024 && ncols <= 256 ? 6 : 5) : WG == 512 && L < 2048 ? 5 : 2;
     if (sign < 0)
-        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, Divider(ncols), total,
-                           in_hint, out_hint, win);
+        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, in_hint,
+                           out_hint, win);
     else
-        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, wab, ncols, Divider(ncols), total,
-                           in_hint, out_hint, win);
+        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, in_hint,
+                           out_hint, win);
     return hipGetLastError();
 }
 
@@ -283,8 +280,8 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, con
 // us against 55.7 at 512, 2048 x 1024 x 8: 55.0 against 75.9).  The lines below
 // are where the measurements leave this rule.
 template <int L>
-hipError_t launch_wide(const float2* in, float2* out, const float2* tc, const float2* wab, uint32_t ncols,
-                       uint32_t total, bool aligned, bool rows_behind, int sign, hipStream_t s) {
+hipError_t launch_wide(const float2* in, float2* out, const float2* tc, uint32_t ncols, uint32_t total, bool aligned,
+                       bool rows_behind, int sign, hipStream_t s) {
     constexpr uint32_t kOne = 256 * (16384 / L);  // columns of one 512-thread workgroup per CU
     if constexpr (L == 512) {
         // 256 threads: whole-line rows of few columns (512 x 256 x 80 73.0 us
@@ -292,9 +289,9 @@ hipError_t launch_wide(const float2* in, float2* out, const float2* tc, const fl
         // against 66.5), other rows up to three quarters of the resident
         // columns (512 x 999 x 12 20.1 against 18.0, x 16 25.3 against 26.8)
         if (aligned ? ncols <= 256 : total <= 12288)
-            return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
+            return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, sign, s);
     } else if constexpr (L == 4096) {
-        if (total > kOne) return launch_cols_wide<L, 1024>(in, out, tc, wab, ncols, total, aligned, sign, s);
+        if (total > kOne) return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, sign, s);
     } else if (aligned) {
         // narrow matrices, behind the 2-D transform's row pass or in less than
         // a round, run better at 512 threads (2-D 1024 x 128 x 128 90.4 us
@@ -302,16 +299,16 @@ hipError_t launch_wide(const float2* in, float2* out, const float2* tc, const fl
         // 51.8; 1024 x 128 x 48 39.9 against 41.5)
         const bool narrow = ncols < 256 && (total < 2 * kOne || (L == 1024 && rows_behind));
         if (total > kOne && !narrow)
-            return launch_cols_wide<L, 1024>(in, out, tc, wab, ncols, total, aligned, sign, s);
+            return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, sign, s);
     } else if (L == 1024 && total <= 6144) {
         // (1024 x 999 x 6 21.4 us against 22.3 at 512 threads, x 7 32.6 against 26.6)
-        return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
+        return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, sign, s);
     }
     // (2048 points: 512 threads from half a round, 2-D 2048 x 256 x 4 23.2 us
     // against 24.0, x 2 22.2 against 20.2)
     if (L == 4096 || total >= kOne / (L == 2048 && aligned ? 2 : 1))
-        return launch_cols_wide<L, 512>(in, out, tc, wab, ncols, total, aligned, sign, s);
-    if constexpr (L < 4096) return launch_cols_wide<L, 256>(in, out, tc, wab, ncols, total, aligned, sign, s);
+        return launch_cols_wide<L, 512>(in, out, tc, ncols, total, aligned, sign, s);
+    if constexpr (L < 4096) return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, sign, s);
     return hipErrorInvalidValue;
 }
 
@@ -368,7 +365,7 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
             // needs to fill the chip: 512 x 64 x 4 5.7 us against 6.3, 512 x
             // 64 x 128 11.6 against 12.7 (512 x 64 x 256: 26.4 against 23.1)
             if (al && F < 12288) return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, sign, s);
-            return launch_wide<512>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
+            return launch_wide<512>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
         case 1024:
             // whole-line rows, more columns than 256-thread workgroups take in
             // one per CU and fewer than 512-thread ones: 2-D 1024 x 1024 x 3
@@ -376,18 +373,17 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
             // and 26.1, 1024 x 64 x 40 23.2 against 24.6 and 27.0
             if (al && F > 2048 && F < 4096)
                 return launch_cols<idx(1024), false, 1024>(i2, o2, t1, nullptr, cv, sign, s);
-            return launch_wide<1024>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
-        case 2048: return launch_wide<2048>(i2, o2, t1, nullptr, ncols, F, al, rows_behind, sign, s);
+            return launch_wide<1024>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
+        case 2048: return launch_wide<2048>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
         default: break;
     }
-    const float2* wab = tc + L.wab;
-    if (F >= kOnePassCols) return launch_wide<4096>(i2, o2, t1, wab, ncols, F, al, rows_behind, sign, s);
+    if (F >= kOnePassCols) return launch_wide<4096>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
     // P-point pass with the twiddle: in -> ws; Q-point pass with the row map: ws -> out
     float2* ws = reinterpret_cast<float2*>(work);
     const uint32_t qn = L.q * ncols;
     const bool whole = line_aligned(in, ws, qn);
     const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, whole ? 0 : 1, whole ? kAutoWindow : kColWindow, {}, {}};
-    hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, wab, a, sign, s);
+    hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, tc + L.wab, a, sign, s);
     if (e != hipSuccess) return e;
     // (with the hint from 16 columns however the rows start: read without it,
     // the lines of the workspace slow the next call's first pass, as above:

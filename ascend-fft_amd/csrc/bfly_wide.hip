@@ -24,14 +24,12 @@ using namespace bfly_dev;
 
 namespace {
 
-// The plan of one length and its LDS twiddles: [second pass's table, stored
-// r R0 + k | W_N^j, j < LO | W_N^{LO j}].
+// The plan of one length; T1: entries of the second pass's table (r R0 + k).
 template <int N>
 struct WidePlan {
     static constexpr int R0 = N == 32768 ? 32 : 16, R1 = N == 8192 ? 16 : 32, R2 = 32;
     static_assert(R0 * R1 * R2 == N, "three passes");
-    static constexpr int LO = N == 8192 ? 64 : N == 16384 ? 128 : 256, HI = N / LO;
-    static constexpr int T1 = R0 * R1, LEN = T1 + LO + HI;
+    static constexpr int T1 = R0 * R1;
 };
 
 // Staggered start.  All resident workgroups begin a launch together, load at
@@ -60,7 +58,8 @@ __global__ __launch_bounds__(N / kWide) __attribute__((amdgpu_waves_per_eu(4, 4)
     using W = WidePlan<N>;
     constexpr int T = N / kWide;
     __shared__ float lds[lds_len(N)];
-    __shared__ float2 tab[W::LEN];
+    __shared__ float2 t1[W::T1];
+    __shared__ Wide64 tab[kWideTab<N>];
     if (blockIdx.x < Stagger<N>::kResident)
         for (uint32_t i = ((blockIdx.x >> Stagger<N>::SHIFT) & Stagger<N>::MASK) * step; i > 0; i--)
             __builtin_amdgcn_s_sleep(2);
@@ -71,11 +70,10 @@ __global__ __launch_bounds__(N / kWide) __attribute__((amdgpu_waves_per_eu(4, 4)
     for (int m = 0; m < kWide / W::R0; m++)
 #pragma unroll
         for (int r = 0; r < W::R0; r++) v[m * W::R0 + r] = ld_stream(&src[t + m * T + r * (N / W::R0)]);
-    float2 *t1 = tab, *tlo = tab + W::T1, *thi = tlo + W::LO;
     for (int i = t; i < W::T1; i += T) t1[i] = wN[(i / W::R0) * (i % W::R0) * (N / W::T1)];
-    for (int i = t; i < W::LO + W::HI; i += T) tlo[i] = wN[i < W::LO ? i : (i - W::LO) * W::LO];
+    wide_table<N>(tab, t);
     // (the first exchange's barriers order the tables before their first read)
-    stockham_wide<N, T, DIR, W::LO, W::R0, 1, W::R0, W::R1, W::R2>(v, lds, tlo, thi, t1, t);
+    stockham_wide<N, T, DIR, W::R0, 1, W::R0, W::R1, W::R2>(v, lds, tab, t1, t);
     if (scale != 1.0f) {  // uniform: the normalised entry point only
 #pragma unroll
         for (int i = 0; i < kWide; i++) v[i] = make_float2(v[i].x * scale, v[i].y * scale);

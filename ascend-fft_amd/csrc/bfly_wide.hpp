@@ -105,65 +105,90 @@ __device__ __forceinline__ void exchange(float2 (&v)[kWide], float* lds, int t) 
 }
 
 // The twiddles of one butterfly, W_{Ns R}^{r k}.  `t1` holds the second
-// pass's table stored [r Ns + k]; later passes combine the two-level tables
-// tlo (W_N^j, j < LO) and thi (W_N^{LO j}).  A radix-32 pass takes ten of its
-// 31 twiddles from them and forms the others as one product more (three
-// lookups and products three deep instead: 4096-point error 1.29e-7 ->
-// 1.49e-7, the same time).
-template <int N, int LO>
-__device__ __forceinline__ float2 tw_lo_hi(const float2* tlo, const float2* thi, int m) {
-    const float2 a = tlo[m & (LO - 1)], b = thi[m / LO];
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+// pass's table stored [r Ns + k].  The third pass forms its 31 as powers of
+// one, W_N^k, in FP64, whose multiply-adds issue at the rate of the FP32 ones
+// here, and rounds each once.  As FP32 products of table entries (ten of two
+// entries, the others of two such products) they added to the transform's
+// error (relative L2 at 8192 / 16384 / 32768 points 1.362e-7 / 1.418e-7 /
+// 1.486e-7; the kernels of 16 points per thread and the four-step chain have
+// 1.315e-7 / 1.416e-7 / 1.414e-7; columns of 4096 points 1.381e-7 against
+// 1.291e-7 in two passes).  So 1.294e-7 / 1.359e-7 / 1.432e-7 and 1.230e-7, in
+// the same time or less (8192 x 512 14.1 -> 13.6 us, 32768 x 256 32.9 -> 32.7).
+struct Wide64 {
+    double x, y;
+};
+__device__ __forceinline__ Wide64 mul64(Wide64 a, Wide64 b) {
+    return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
+// W_L^m
+__device__ __forceinline__ Wide64 root64(int m, int L) {
+    Wide64 w;
+    sincospi(-2.0 * m / L, &w.y, &w.x);
+    return w;
+}
+// W_N^k = tab[k % kWideLo] tab[kWideLo + k / kWideLo], k < N / 32.
+constexpr int kWideLo = 32;
+template <int N>
+constexpr int kWideTab = kWideLo + N / kWide / kWideLo;
+template <int N>
+__device__ __forceinline__ void wide_table(Wide64* tab, int tid) {
+    if (tid < kWideTab<N>) tab[tid] = root64(tid < kWideLo ? tid : (tid - kWideLo) * kWideLo, N);
+}
+// 32768 points multiply by the unrounded twiddles as well: the four-step chain
+// reads all of its own from tables (1.432e-7 -> 1.405e-7; 8192 x 2048 would
+// take 49.2 us instead of 48.5).
+template <int N>
+constexpr bool kProduct64 = N == 32768;
 // Multiplies the MM butterflies v[m R ..] that share one k.
-template <int N, int LO, int DIR, int First, int Ns, int R, int MM>
-__device__ __forceinline__ void wide_twiddle(float2* v, const float2* tlo, const float2* thi, const float2* t1,
-                                             int k) {
-    auto apply = [&](int r, float2 w) {
-#pragma unroll
-        for (int m = 0; m < MM; m++) v[m * R + r] = cmul_tw<DIR>(v[m * R + r], w);
-    };
+template <int N, int DIR, int First, int Ns, int R, int MM>
+__device__ __forceinline__ void wide_twiddle(float2* v, const Wide64* tab, const float2* t1, int k) {
     if constexpr (Ns == First) {
 #pragma unroll
-        for (int r = 1; r < R; r++) apply(r, t1[r * Ns + k]);
+        for (int r = 1; r < R; r++)
+#pragma unroll
+            for (int m = 0; m < MM; m++) v[m * R + r] = cmul_tw<DIR>(v[m * R + r], t1[r * Ns + k]);
     } else {
-        static_assert(R == 32, "only radix 32 follows the second pass");
-        // W^{r e}, r = 4 a + b, as W^{4 a e} W^{b e}: few live at a time
-        const int e = k * (N / (Ns * R));
-        auto mul = [](float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
-        float2 w[4];
+        static_assert(R == 32 && MM == 1 && Ns * R == N, "only a last radix-32 pass follows the second");
+        // W^{r k} for r = b, b + 4, ..: few live at a time
+        const Wide64 w1 = mul64(tab[k % kWideLo], tab[kWideLo + k / kWideLo]), w2 = mul64(w1, w1),
+                     w4 = mul64(w2, w2);
+        Wide64 first = w1;
 #pragma unroll
-        for (int b = 1; b < 4; b++) {
-            w[b] = tw_lo_hi<N, LO>(tlo, thi, b * e);
-            apply(b, w[b]);
-        }
+        for (int b = 1; b <= 4; b++) {
+            Wide64 w = first;
 #pragma unroll
-        for (int a = 1; a < 8; a++) {
-            const float2 p = tw_lo_hi<N, LO>(tlo, thi, 4 * a * e);
-            apply(4 * a, p);
-#pragma unroll
-            for (int b = 1; b < 4; b++) apply(4 * a + b, mul(p, w[b]));
+            for (int r = b; r < R; r += 4) {
+                if constexpr (kProduct64<N>) {
+                    const Wide64 p = mul64({v[r].x, v[r].y}, {w.x, DIR < 0 ? w.y : -w.y});
+                    v[r] = make_float2((float)p.x, (float)p.y);
+                } else {
+                    v[r] = cmul_tw<DIR>(v[r], make_float2((float)w.x, (float)w.y));
+                }
+                if (r + 4 < R) w = mul64(w, w4);
+            }
+            if (b < 4) first = mul64(first, w1);
         }
     }
 }
 
 // Runs passes <R, Rest...> with Ns points combined; on entry v[m R + r] =
 // x[t + m T + r N/R], on exit v[m RL + r] = X[t + m T + r N/RL].  First = the
-// first pass's radix; `lds` = this transform's lds_len(N) floats.  Every LDS
-// read has ended (a barrier passed) when an exchange returns.
-template <int N, int T, int DIR, int LO, int First, int Ns, int R, int... Rest>
-__device__ __forceinline__ void stockham_wide(float2 (&v)[kWide], float* lds, const float2* tlo, const float2* thi,
-                                              const float2* t1, int t) {
+// first pass's radix; `lds` = this transform's lds_len(N) floats; `tab`: of
+// wide_table, unused by two passes.  Every LDS read has ended (a barrier
+// passed) when an exchange returns.
+template <int N, int T, int DIR, int First, int Ns, int R, int... Rest>
+__device__ __forceinline__ void stockham_wide(float2 (&v)[kWide], float* lds, const Wide64* tab, const float2* t1,
+                                              int t) {
     static_assert(kWide % R == 0 && N == T * kWide, "32 points per thread");
     constexpr int M = kWide / R;
     if constexpr (Ns > 1 && T % Ns == 0) {
         // every butterfly of the thread has the same k
-        wide_twiddle<N, LO, DIR, First, Ns, R, M>(v, tlo, thi, t1, t & (Ns - 1));
+        wide_twiddle<N, DIR, First, Ns, R, M>(v, tab, t1, t & (Ns - 1));
     }
 #pragma unroll
     for (int m = 0; m < M; m++) {
         if constexpr (Ns > 1 && T % Ns != 0)
-            wide_twiddle<N, LO, DIR, First, Ns, R, 1>(&v[m * R], tlo, thi, t1, (t + m * T) & (Ns - 1));
+            wide_twiddle<N, DIR, First, Ns, R, 1>(&v[m * R], tab, t1, (t + m * T) & (Ns - 1));
         dft<R, DIR>(&v[m * R]);
         // one butterfly at a time: interleaved, their temporaries spill
         __builtin_amdgcn_sched_barrier(0);
@@ -173,7 +198,7 @@ __device__ __forceinline__ void stockham_wide(float2 (&v)[kWide], float* lds, co
         constexpr int R2 = bfly_dev::First<Rest...>::value;
         exchange<N, T, Ns, R, R2>(v, lds, t);
         asm volatile("" : "+v"(t));
-        stockham_wide<N, T, DIR, LO, First, Ns * R, Rest...>(v, lds, tlo, thi, t1, t);
+        stockham_wide<N, T, DIR, First, Ns * R, Rest...>(v, lds, tab, t1, t);
     }
 }
 
