@@ -35,7 +35,8 @@ def supported(kind: int, n: int) -> bool:
 
 def table(kind: int, n: int, device) -> torch.Tensor:
     """Device copy of the FP64-generated twiddle table of (kind, n), cached."""
-    device = torch.device(device)
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
     key = (device.index, kind, n)
     t = _tables.get(key)
     if t is None:
@@ -132,7 +133,9 @@ def c2c(x: torch.Tensor, sign: int = -1, norm: str | None = None, *, scale: floa
     if batch == 0:
         return out
     factor = norm_scale(n, sign, norm) if scale is None else scale
-    c2c_raw(plain(x), out, n, batch, sign, scale=None if factor == 1.0 else factor)
+    if x.is_neg():
+        x = plain(x)
+    c2c_raw(x, out, n, batch, sign, scale=None if factor == 1.0 else factor)
     return out
 
 
@@ -241,7 +244,8 @@ def fft2(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
 
 def _real(kind: int, src: torch.Tensor, dst: torch.Tensor, n: int, batch: int, bins: int, stride: int,
           adjoint: bool, what: str) -> None:
-    src = plain(src)
+    if src.is_neg():
+        src = plain(src)
     tab = table(kind, n, src.device)
     rc = _lib.hip().bfly_real_ex(kind, src.data_ptr(), dst.data_ptr(), n, batch, bins, stride,
                                  _lib.VARIANT_AUTO, _lib.REAL_ADJOINT if adjoint else 0, tab.data_ptr(),

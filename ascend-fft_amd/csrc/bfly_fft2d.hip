@@ -3,10 +3,12 @@
 //
 // X[k1][k2] = sum_{j1, j2} x[j1][j2] W_n1^{j1 k1} W_n2^{j2 k2} is separable:
 // the row pass is the C2C kernels over batch * n1 rows of n2 points; the
-// column pass takes C adjacent columns per workgroup, so that every load and
-// store is a run of C consecutive complex values.  Columns are numbered
-// through the batch, so a group may span two items and no lane idles where
-// the columns per item are few or no multiple of C.  Two kernels:
+// column pass takes up to C columns per workgroup, so that every load and
+// store is a run of consecutive complex values.  Matrices of C columns and
+// their multiples are cut into groups of C; narrower ones go whole into a
+// group; the columns of other widths are numbered through the batch, so that
+// a group may span two matrices and no lane idles (bfly_columns.hpp).  Two
+// kernels:
 //
 //   k_cols       16 points per thread, up to 256-point columns (and 512- and
 //                1024-point ones in few groups): C >= 16;
@@ -26,6 +28,7 @@
 
 #include <cstdint>
 
+#include "bfly_columns.hpp"
 #include "bfly_hip.h"
 #include "bfly_kernels.hpp"
 #include "bfly_tables.hpp"
@@ -35,6 +38,7 @@
 namespace {
 
 using namespace bfly_dev;
+using namespace bfly_cols;
 
 // Addressing of one column pass.  A batch item of `item` elements holds
 // `mats` matrices of `ncols` columns; matrix m of item b reads rows at
@@ -49,8 +53,9 @@ struct ColView {
     uint32_t col_div;  // twiddle pass: q = column / col_div
     int temporal;      // without the streaming hint (line_aligned)
     uint32_t win;      // log2 of the units per XCD window (kAutoWindow: the launcher's choice)
-    Divider unit;      // set by the launcher: by the groups per matrix if whole, else by its columns
-    Divider mat;       // set by the launcher: by mats
+    uint32_t per;      // set by the launcher, as what follows: columns per workgroup
+    Divider unit;      // by the groups per matrix if whole, else by its columns
+    Divider mat;       // by mats
 };
 
 // Rows that start on 128-byte lines: a run of 16 or more columns then covers
@@ -58,9 +63,10 @@ struct ColView {
 // 53.3 without it).  Other rows share every line with the neighbouring
 // columns' workgroup, which the L2 serves and merges only without the hint
 // (512 x 1001 x 24, windows of 8: 50.8 us against 76.4 with it).
-bool line_aligned(const void* in, const void* out, uint32_t ncols) {
-    return ncols % 16 == 0 && (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 128 == 0;
+bool on_lines(const void* in, const void* out) {
+    return (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 128 == 0;
 }
+bool line_aligned(const void* in, const void* out, uint32_t ncols) { return ncols % 16 == 0 && on_lines(in, out); }
 
 // Units per XCD window (xcd_window) of the column kernels.  Sweep 1 / 2 / 4 /
 // 8 / 16 / 64 of the 16-point kernel: 512 x 1001 x 24 66.6 / 58.3 / 53.1 /
@@ -74,12 +80,12 @@ constexpr uint32_t kAutoWindow = ~0u;
 // 45.8; 512 of them: 17.8 against 14.1).
 constexpr uint32_t kOnePassCols = 1024;
 
-// One column group per workgroup: C = WG / T adjacent columns, 16 points per
-// thread.  Bound by HBM (run lengths of C columns); columns up to 256 points,
-// and 512-point ones in few groups (column_pass).
+// One column group per workgroup: C = WG / T columns, 16 points per thread.
+// Bound by HBM (run lengths of C columns); columns up to 256 points, and
+// 512- and 1024-point ones in few groups (column_pass).
 // HINT: streaming accesses (a template argument: both forms in one kernel cost
 // a launch 0.1 us more, 256 x 256 x 8 5.04 -> 4.95).
-template <int I, int DIR, bool TW, int WG, bool HINT>
+template <int I, int DIR, bool TW, int WG, bool HINT, bool WHOLE, Order ORDER>
 __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ wab,
                                               ColView cv) {
@@ -95,19 +101,35 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
     __shared__ float2 ltw[LT::LEN];
     __shared__ float2 wt[TW ? 128 : 1];
     const int tid = threadIdx.x;
-    // the column plan's tables, [its pass tables | A | B] as in the local C2C
-    // table: fetched ahead of the columns, parked in LDS behind their loads
+    constexpr bool FIRST = ORDER == kFirst || ORDER == kFirstGuard, GUARD = ORDER == kFirstGuard || ORDER == kAheadGuard;
+    // the column plan's tables: [its pass tables | A | B] as in the local C2C table
+    const float2* ab = tw + bfly_plan::stage_twiddle_len(I);
     C2cLdsTwFetch<I, WG> tabs;
-    tabs.fetch(tw, tw + bfly_plan::stage_twiddle_len(I), tid);
+    auto stage = [&] {
+        if constexpr (FIRST) c2c_lds_tw<I, WG>(ltw, tw, ab, tid);
+        else tabs.park(ltw, tid);
+        if constexpr (TW)
+            for (int i = tid; i < 128; i += WG) wt[i] = wab[i];
+    };
+    if constexpr (FIRST) stage();
+    else tabs.fetch(tw, ab, tid);
     const int c = tid % C, t = tid / C;
-    const uint32_t blk = xcd_window_log2(blockIdx.x, gridDim.x, cv.win), f = blk * C + c;
-    const bool active = f < cv.total;
+    const uint32_t blk = xcd_window_log2(blockIdx.x, gridDim.x, cv.win);
     uint32_t mi, col;  // matrix and column of this lane
-    if (cv.ncols % C == 0) {  // whole groups: one division per workgroup
+    bool active;
+    if constexpr (WHOLE) {
         mi = cv.unit.divide(blk, &col);
         col = col * C + c;
+        active = !GUARD || col < cv.ncols;
     } else {
-        mi = cv.unit.divide(f, &col);
+        const uint32_t f0 = blk * cv.per, f = f0 + c;
+        active = (uint32_t)c < cv.per && f < cv.total;
+        if constexpr (GUARD) {
+            mi = cv.unit.divide(f, &col);
+        } else {
+            const uint32_t last = (cv.per < cv.total - f0 ? f0 + cv.per : cv.total) - 1;
+            mi = cv.unit.divide(active ? f : last, &col);  // reads the last column again
+        }
     }
     uint32_t b = mi, m = 0;
     if (cv.mats > 1) b = cv.mat.divide(mi, &m);
@@ -116,12 +138,11 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
 #pragma unroll
     for (int mm = 0; mm < P / R0; mm++)
 #pragma unroll
-        for (int r = 0; r < R0; r++)
-            v[mm * R0 + r] = active ? ld_io<HINT>(&src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))])
-                                    : make_float2(0.f, 0.f);
-    tabs.park(ltw, tid);
-    if constexpr (TW)
-        for (int i = tid; i < 128; i += WG) wt[i] = wab[i];
+        for (int r = 0; r < R0; r++) {
+            const float2* p = &src[(uint64_t)cv.in_rstride * (t + mm * T + r * (L / R0))];
+            v[mm * R0 + r] = !GUARD || active ? ld_io<HINT>(p) : make_float2(0.f, 0.f);
+        }
+    if constexpr (!FIRST) stage();
     // the transform's first LDS exchange orders the table writes before any read
     run_plan_lt<I, T, DIR, LX_PAD>(v, lds + c * STRIDE, 0, ltw, ltw + LT::NLO, ltw + LT::NLO + LT::NHI, t,
                                    std::make_index_sequence<PL::NRAD>{});
@@ -186,7 +207,7 @@ __device__ __forceinline__ float2 col_root(const float2* __restrict__ tc, int m)
 template <int L, int DIR, int WG>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_cols_wide(
     const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tc, uint32_t ncols,
-    Divider cols, uint32_t total, int stream_in, int stream_out, uint32_t win) {
+    Divider cols, uint32_t total, uint32_t per, int stream_in, int stream_out, uint32_t win) {
     using P = ColPlan<L>;
     constexpr int T = L / kWide, C = WG / T;
     // columns lie 32 / C banks apart (mod 64), so that the C columns and the
@@ -200,9 +221,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     const int tid = threadIdx.x;
     const int c = tid % C;
     int t = tid / C;
-    // columns are numbered through the batch (f = item * ncols + column)
-    const uint32_t f = xcd_window_log2(blockIdx.x, gridDim.x, win) * C + c;
-    const uint32_t fr = f < total ? f : total - 1;  // past the end: reads the last column again
+    // columns are numbered through the batch (f = item * ncols + column), `per`
+    // of them to a workgroup
+    const uint32_t f0 = xcd_window_log2(blockIdx.x, gridDim.x, win) * per, f = f0 + c;
+    const uint32_t end = per < total - f0 ? f0 + per : total;
+    const uint32_t fr = f < end ? f : end - 1;  // beyond: reads the last column again
     uint32_t col;
     const uint32_t item = cols.divide(fr, &col);
     const uint64_t at = (uint64_t)item * L * ncols + col;
@@ -226,7 +249,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     } else {
         stockham_wide<L, T, DIR, P::R0, 1, P::R0, P::R1>(v, lds + c * STRIDE, tab, t1, t);
     }
-    if (f >= total) return;
+    if (f >= end) return;
     constexpr int RL = P::R2 > 1 ? P::R2 : P::R1;
     asm volatile("" : "+v"(t));
     float2* dst = out + (at + (uint64_t)t * ncols);
@@ -243,9 +266,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 
 template <int L, int WG>
 hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, uint32_t ncols, uint32_t total,
-                            bool aligned, int sign, hipStream_t s) {
-    constexpr uint32_t C = WG / (L / kWide);
-    const uint32_t blocks = (uint32_t)(((uint64_t)total + C - 1) / C);
+                            bool aligned, bool on_line, int sign, hipStream_t s) {
+    const Grid grid = column_grid(WG / (L / kWide), L, ncols, total, false, true);
+    const uint32_t per = grid.per, blocks = grid.blocks;
     // Access hints and windows (kColWindow: why windows; line_aligned: why
     // other rows stay without hints).  Whole-line rows take the streaming
     // hint on the input: read into the L2s without it, the lines of a buffer
@@ -256,16 +279,17 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, uin
     // 2048 points and 512 threads (2-D 2048 x 256 x 4: 22.5 against 24.1);
     // so are 1024-point ones in one round of workgroups (1024 x 256 x 32:
     // 26.9 against 29.1).
-    const int in_hint = aligned;
-    const int out_hint = aligned && (L == 512 || (L == 1024 && (WG < 1024 || blocks >= 512)) || (L == 2048 && WG == 512));
+    const int own = grid.own && on_line;
+    const int in_hint = aligned || own;
+    const int out_hint = (own && !aligned) || (aligned && (L == 512 || (L == 1024 && (WG < 1024 || blocks >= 512)) || (L == 2048 && WG == 512)));
     // (log2 of the window)
     const uint32_t win = !aligned ? 5 : WG == 1024 ? (L == 1024 && ncols <= 256 ? 6 : 5) : WG == 512 && L < 2048 ? 5 : 2;
     if (sign < 0)
-        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, in_hint,
-                           out_hint, win);
+        hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, per,
+                           in_hint, out_hint, win);
     else
-        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, in_hint,
-                           out_hint, win);
+        hipLaunchKernelGGL((k_cols_wide<L, 1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, per,
+                           in_hint, out_hint, win);
     return hipGetLastError();
 }
 
@@ -281,17 +305,33 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, uin
 // are where the measurements leave this rule.
 template <int L>
 hipError_t launch_wide(const float2* in, float2* out, const float2* tc, uint32_t ncols, uint32_t total, bool aligned,
-                       bool rows_behind, int sign, hipStream_t s) {
+                       bool on_line, bool rows_behind, int sign, hipStream_t s) {
     constexpr uint32_t kOne = 256 * (16384 / L);  // columns of one 512-thread workgroup per CU
+    constexpr uint32_t C512 = 16384 / L;          // columns of a 512-thread workgroup
+    // Matrices narrower than a line, once smaller workgroups would give each CU
+    // one: the smallest that holds a matrix (bfly_columns.hpp; 1024 x 12 x 400 24.2 ->
+    // 17.1 us, 2048 x 7 x 300 24.4 -> 16.7; below, 1024 x 12 x 50 8.2 against 10.0),
+    // or two that fill it (1024 x 8 x 1000 26.0 -> 21.6)
+    if (ncols < 16) {
+        const uint32_t mats = total / ncols;
+        if constexpr (L < 4096)
+            if (2 * ncols <= C512 && !(2 * ncols == C512 && mats > 768))
+                return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, on_line, sign, s);
+        if constexpr (L > 512)
+            if (ncols > C512 && total > 192 * C512)
+                return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, on_line, sign, s);
+        if (ncols <= C512 && total > 96 * C512)
+            return launch_cols_wide<L, 512>(in, out, tc, ncols, total, aligned, on_line, sign, s);
+    }
     if constexpr (L == 512) {
         // 256 threads: whole-line rows of few columns (512 x 256 x 80 73.0 us
         // against 65.5 at 512 threads, x 128 105 against 99; 512 columns 63.5
         // against 66.5), other rows up to three quarters of the resident
         // columns (512 x 999 x 12 20.1 against 18.0, x 16 25.3 against 26.8)
         if (aligned ? ncols <= 256 : total <= 12288)
-            return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, sign, s);
+            return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, on_line, sign, s);
     } else if constexpr (L == 4096) {
-        if (total > kOne) return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, sign, s);
+        if (total > kOne) return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, on_line, sign, s);
     } else if (aligned) {
         // narrow matrices, behind the 2-D transform's row pass or in less than
         // a round, run better at 512 threads (2-D 1024 x 128 x 128 90.4 us
@@ -299,36 +339,76 @@ hipError_t launch_wide(const float2* in, float2* out, const float2* tc, uint32_t
         // 51.8; 1024 x 128 x 48 39.9 against 41.5)
         const bool narrow = ncols < 256 && (total < 2 * kOne || (L == 1024 && rows_behind));
         if (total > kOne && !narrow)
-            return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, sign, s);
+            return launch_cols_wide<L, 1024>(in, out, tc, ncols, total, aligned, on_line, sign, s);
     } else if (L == 1024 && total <= 6144) {
         // (1024 x 999 x 6 21.4 us against 22.3 at 512 threads, x 7 32.6 against 26.6)
-        return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, sign, s);
+        return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, on_line, sign, s);
     }
     // (2048 points: 512 threads from half a round, 2-D 2048 x 256 x 4 23.2 us
     // against 24.0, x 2 22.2 against 20.2)
     if (L == 4096 || total >= kOne / (L == 2048 && aligned ? 2 : 1))
-        return launch_cols_wide<L, 512>(in, out, tc, ncols, total, aligned, sign, s);
-    if constexpr (L < 4096) return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, sign, s);
+        return launch_cols_wide<L, 512>(in, out, tc, ncols, total, aligned, on_line, sign, s);
+    if constexpr (L < 4096) return launch_cols_wide<L, 256>(in, out, tc, ncols, total, aligned, on_line, sign, s);
     return hipErrorInvalidValue;
 }
 
 template <int I, bool TW, int WG = bfly_plan::kBlock>
-hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const float2* wab, ColView cv, int sign,
-                       hipStream_t s) {
+hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const float2* wab, ColView cv, bool on_line,
+                       int sign, hipStream_t s) {
     constexpr uint32_t C = WG / PlanOf<I>::T;
-    const uint32_t blocks = (uint32_t)(((uint64_t)cv.total + C - 1) / C);
-    // whole-line rows in a round of workgroups or less: as dealt (the split's
-    // first pass at 4096 x 64 x 4 5.4 us against 6.6); 64 and 128 points
-    // always (128 x 2048 x 64 46.2 us against 59.0 in windows, other widths equal)
     constexpr int L = PlanOf<I>::N;
-    if (cv.win == kAutoWindow) cv.win = blocks >= 1024 && L != 64 && L != 128 ? kColWindow : 0;
-    cv.unit = Divider(cv.ncols % C == 0 ? cv.ncols / C : cv.ncols);
+    // (a pass of the split reads or writes rows that its matrices share)
+    const bool split = TW || cv.mats > 1;
+    const Grid grid = column_grid(C, L, cv.ncols, cv.total, true, !split);
+    const bool whole = grid.whole;
+    const uint32_t blocks = grid.blocks;
+    cv.per = grid.per;
+    if (grid.own && on_line) cv.temporal = 0;
+    // whole-line rows in fewer workgroups: as dealt (the split's first pass at
+    // 4096 x 64 x 4 5.4 us against 6.6; 256 x 64 x 256 13.6 against 14.1); 64 and 128 points
+    // always (128 x 2048 x 64 46.2 us against 59.0 in windows, other widths equal)
+    if (cv.win == kAutoWindow) cv.win = blocks >= 2048 && L != 64 && L != 128 ? kColWindow : 0;
+    cv.unit = Divider(whole ? cv.ncols / C : cv.ncols);
     cv.mat = Divider(cv.mats);
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+    auto go = [&](auto hint, auto w, auto order) {
+        constexpr bool H = decltype(hint)::value, W = decltype(w)::value;
+        constexpr Order O = decltype(order)::value;
+        if (sign < 0)
+            hipLaunchKernelGGL((k_cols<I, -1, TW, WG, H, W, O>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
+        else
+            hipLaunchKernelGGL((k_cols<I, 1, TW, WG, H, W, O>), dim3(blocks), dim3(WG), 0, s, in, out, tw, wab, cv);
     };
-    if (cv.temporal) sign < 0 ? go(&k_cols<I, -1, TW, WG, false>) : go(&k_cols<I, 1, TW, WG, false>);
-    else sign < 0 ? go(&k_cols<I, -1, TW, WG, true>) : go(&k_cols<I, 1, TW, WG, true>);
+    auto pick = [&](auto w, auto order) {
+        if (cv.temporal) go(std::false_type{}, w, order);
+        else go(std::true_type{}, w, order);
+    };
+    constexpr std::integral_constant<Order, kFirst> first{};
+    constexpr std::integral_constant<Order, kFirstGuard> first_guard{};
+    if (!whole) {
+        // ragged groups: tables ahead, at 16 and 32 points guarded (16 x 1000
+        // x 400 22.5 us against 23.7, 256 x 1001 x 48 44.0 against 42.5 at
+        // 256); matrices by themselves as whole groups at their workgroup counts
+        constexpr std::integral_constant<Order, kAheadGuard> ahead_guard{};
+        constexpr std::integral_constant<Order, L <= 32 ? kAheadGuard : kAhead> ragged{};
+        if (grid.own && blocks * (WG / 256) > 512 && blocks * (WG / 256) <= 1024) pick(std::false_type{}, first_guard);
+        else if (L == 64 && split && blocks > 512) pick(std::false_type{}, ahead_guard);  // as below
+        else pick(std::false_type{}, ragged);
+        return hipGetLastError();
+    }
+    // (the split's passes: 4096 x 5 x 200 25.9 us against 27.2 tables first, 29.8 unguarded)
+    const Order order = split && blocks > 512 ? kAheadGuard : whole_order(L, blocks * (WG / 256));
+    if constexpr (L <= 128)
+        if (order == kAhead) {
+            pick(std::true_type{}, std::integral_constant<Order, kAhead>{});
+            return hipGetLastError();
+        }
+    if constexpr (L == 64 || L == 128)
+        if (order == kAheadGuard) {
+            pick(std::true_type{}, std::integral_constant<Order, kAheadGuard>{});
+            return hipGetLastError();
+        }
+    if (order == kFirstGuard) pick(std::true_type{}, first_guard);
+    else pick(std::true_type{}, first);
     return hipGetLastError();
 }
 
@@ -345,53 +425,54 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
     // workgroup counts fit 32 bits
     if (total == 0 || total > 0x7fffffffull) return hipErrorInvalidValue;
     const uint32_t F = (uint32_t)total;
-    const bool al = line_aligned(in, out, ncols);
+    const bool on_line = on_lines(in, out), al = line_aligned(in, out, ncols);
     constexpr auto idx = bfly_plan::plan_index;
     // (16 and 32 points, whose runs of 2 and 1 KiB are mostly whole lines
     // however the rows start, past what the last-level cache holds: 16 x 1000
     // x 700 32.6 us with the hint, 34.7 without; 16 x 1000 x 400 20.4 against
     // 17.2, 32 x 167 x 500 11.6 against 9.3)
     const bool hint = al || (n1 <= 32 && item * batch > (1ull << 23));
-    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, hint ? 0 : 1, al ? kAutoWindow : kColWindow, {}, {}};
+    const ColView cv{item, 0, 0, ncols, ncols, ncols, 1, F, 1, hint ? 0 : 1, al ? kAutoWindow : kColWindow, 0, {}, {}};
     const float2* t1 = tc + L.p_table;
     switch (n1) {
-        case 16: return launch_cols<idx(16), false>(i2, o2, t1, nullptr, cv, sign, s);
-        case 32: return launch_cols<idx(32), false>(i2, o2, t1, nullptr, cv, sign, s);
-        case 64: return launch_cols<idx(64), false>(i2, o2, t1, nullptr, cv, sign, s);
-        case 128: return launch_cols<idx(128), false>(i2, o2, t1, nullptr, cv, sign, s);
-        case 256: return launch_cols<idx(256), false>(i2, o2, t1, nullptr, cv, sign, s);
+        case 16: return launch_cols<idx(16), false>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+        case 32: return launch_cols<idx(32), false>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+        case 64: return launch_cols<idx(64), false>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+        case 128: return launch_cols<idx(128), false>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+        case 256: return launch_cols<idx(256), false>(i2, o2, t1, nullptr, cv, on_line, sign, s);
         case 512:
             // whole-line rows in fewer column groups than the wide kernel
             // needs to fill the chip: 512 x 64 x 4 5.7 us against 6.3, 512 x
             // 64 x 128 11.6 against 12.7 (512 x 64 x 256: 26.4 against 23.1)
-            if (al && F < 12288) return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, sign, s);
-            return launch_wide<512>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
+            // (and narrower than a line: 512 x 8 x 1000 11.6 against 12.4)
+            if ((al && F < 12288) || ncols < 16) return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+            return launch_wide<512>(i2, o2, t1, ncols, F, al, on_line, rows_behind, sign, s);
         case 1024:
             // whole-line rows, more columns than 256-thread workgroups take in
             // one per CU and fewer than 512-thread ones: 2-D 1024 x 1024 x 3
             // 24.2 us against 29.6 and 23.9, 1024 x 128 x 24 23.5 against 29.1
             // and 26.1, 1024 x 64 x 40 23.2 against 24.6 and 27.0
             if (al && F > 2048 && F < 4096)
-                return launch_cols<idx(1024), false, 1024>(i2, o2, t1, nullptr, cv, sign, s);
-            return launch_wide<1024>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
-        case 2048: return launch_wide<2048>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
+                return launch_cols<idx(1024), false, 1024>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+            return launch_wide<1024>(i2, o2, t1, ncols, F, al, on_line, rows_behind, sign, s);
+        case 2048: return launch_wide<2048>(i2, o2, t1, ncols, F, al, on_line, rows_behind, sign, s);
         default: break;
     }
-    if (F >= kOnePassCols) return launch_wide<4096>(i2, o2, t1, ncols, F, al, rows_behind, sign, s);
+    if (F >= kOnePassCols) return launch_wide<4096>(i2, o2, t1, ncols, F, al, on_line, rows_behind, sign, s);
     // P-point pass with the twiddle: in -> ws; Q-point pass with the row map: ws -> out
     float2* ws = reinterpret_cast<float2*>(work);
     const uint32_t qn = L.q * ncols;
     const bool whole = line_aligned(in, ws, qn);
-    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, whole ? 0 : 1, whole ? kAutoWindow : kColWindow, {}, {}};
-    hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, tc + L.wab, a, sign, s);
+    const ColView a{item, 0, 0, qn, qn, qn, 1, qn * batch, ncols, whole ? 0 : 1, whole ? kAutoWindow : kColWindow, 0, {}, {}};
+    hipError_t e = launch_cols<idx(64), true>(i2, ws, t1, tc + L.wab, a, false, sign, s);
     if (e != hipSuccess) return e;
     // (with the hint from 16 columns however the rows start: read without it,
     // the lines of the workspace slow the next call's first pass, as above:
     // 4096 x 60 x 7 14.4 us against 18.5; 4096 x 3 x 214 25.7 against 21.7)
     const bool own = line_aligned(ws, out, ncols);
     const ColView b{item, qn, ncols, ncols, L.p * ncols, ncols, L.p, qn * batch, 1, own || ncols >= 16 ? 0 : 1,
-                    own ? kAutoWindow : kColWindow, {}, {}};
-    return launch_cols<idx(64), false>(ws, o2, tc + L.q_table, nullptr, b, sign, s);
+                    own ? kAutoWindow : kColWindow, 0, {}, {}};
+    return launch_cols<idx(64), false>(ws, o2, tc + L.q_table, nullptr, b, false, sign, s);
 }
 
 }  // namespace

@@ -144,7 +144,11 @@ constexpr int c2c_lds_tw_len() { return C2cLdsTw<I>::NLO + C2cLdsTw<I>::NHI + (k
 template <int I, int WG>
 __device__ __forceinline__ void c2c_lds_tw(float2* buf, const float2* __restrict__ tw,
                                            const float2* __restrict__ ab, int tid) {
-    for (int i = tid; i < c2c_lds_tw_len<I>(); i += WG) buf[i] = c2c_lds_tw_entry<I>(tw, ab, i);
+    using L = C2cLdsTw<I>;
+    for (int i = tid; i < L::NLO + L::NHI; i += WG) buf[i] = ab[i];
+    if constexpr (kPlans[I].nrad > 1)
+        for (int i = tid; i < L::NT1; i += WG)
+            buf[L::NLO + L::NHI + (i % L::R1) * bfly_plan::kPoints + i / L::R1] = tw[i];
 }
 
 // The same in two halves, for a kernel that issues its data loads in
