@@ -424,7 +424,7 @@ int bfly_host_pipelined(int kind, int sign, int variant, const float* host_in, f
             }
             const hipError_t e =
                 kind == BFLY_KIND_C2C
-                    ? bfly_kern::c2c(din, dout, n, rows, sign, variant, table, work, up, nullptr, 1.0f)
+                    ? bfly_kern::c2c(din, dout, n, rows, sign, sh.kernel, table, work, up, nullptr, 1.0f)
                     : bfly_kern::real(kind, din, dout, n, rows, n / 2 + 1, n + 2, variant, false, table, up);
             if (e != hipSuccess) {
                 rc = BFLY_ERR_LAUNCH;
@@ -463,7 +463,7 @@ int bfly_host_pipelined(int kind, int sign, int variant, const float* host_in, f
         }
         const hipError_t e =
             kind == BFLY_KIND_C2C
-                ? bfly_kern::c2c(din, dout, n, rows, sign, variant, table, work, P.comp, nullptr, 1.0f)
+                ? bfly_kern::c2c(din, dout, n, rows, sign, sh.kernel, table, work, P.comp, nullptr, 1.0f)
                 : bfly_kern::real(kind, din, dout, n, rows, n / 2 + 1, n + 2, variant, false, table, P.comp);
         if (e != hipSuccess || hipEventRecord(done, P.comp) != hipSuccess ||
             hipStreamWaitEvent(P.down, done, 0) != hipSuccess) {

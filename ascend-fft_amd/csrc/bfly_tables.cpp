@@ -332,12 +332,17 @@ int check_pipelined(int kind, int sign, int variant, const void* host_in, const 
     if (cr > batch) cr = batch;
     shape->chunk = cr;
     // the kernels run on chunks, so AUTO picks the variant for a chunk's batch
+    int kernel = variant;
     if (c2c) {
-        if (variant == BFLY_VARIANT_AUTO) variant = auto_variant(n, (uint32_t)cr);
+        if (variant == BFLY_VARIANT_AUTO) {
+            variant = auto_variant(n, (uint32_t)cr);
+            kernel = auto_kernel(n, (uint32_t)cr);
+        }
     } else {
         if (variant == BFLY_VARIANT_AUTO) variant = auto_real_variant(n, (uint32_t)cr);
         if (variant != BFLY_VARIANT_PLAIN && variant != BFLY_VARIANT_STREAM && variant != BFLY_VARIANT_STREAM_LT)
             return BFLY_ERR_SHAPE;
+        kernel = variant;
     }
     if (int g = check_execute(kind, sign, dev_in, dev_out, n, batch, table, c2c ? work : nullptr, variant))
         return g;
@@ -352,6 +357,7 @@ int check_pipelined(int kind, int sign, int variant, const void* host_in, const 
     }
     shape->sign = sign;
     shape->variant = variant;
+    shape->kernel = kernel;
     return BFLY_OK;
 }
 

@@ -90,8 +90,10 @@ int auto_real_variant(uint32_t n, uint32_t batch);
 // and the CPU stub): resolves the direction of the real kinds and the AUTO
 // variant for one chunk's batch, checks the whole batch as one execute call
 // on the device buffers, and gives the row sizes (floats) and transforms per chunk.
+// `variant` is the public one, which decides the workspace; `kernel` what runs
+// (auto_kernel's under AUTO).
 struct PipeShape {
-    int sign = -1, variant = 0;
+    int sign = -1, variant = 0, kernel = 0;
     size_t row_in = 0, row_out = 0;
     uint64_t chunk = 0;
 };
