@@ -58,6 +58,7 @@ __device__ __forceinline__ void store_pair(float2* p, float4 c) {
 constexpr int kKT = 8;  // modes per workgroup, one per wave
 constexpr int kRT = 8;  // reduction chunk: two 4-deep matrix steps
 constexpr int kThreads = 64 * kKT;
+constexpr uint64_t kMaxGridX = 1u << 22;
 
 // LDS layout of a chunk: [r][row][4 slots of two modes], where modes 2 p, 2 p
 // + 1 of (r, row) are in slot p ^ (row / 4 % 4), swapped for odd r: the 16
@@ -267,15 +268,17 @@ __global__ __launch_bounds__(kThreads) void k_mix(const float2* __restrict__ A, 
                                                   float2* __restrict__ C, uint32_t M, uint32_t N, uint32_t R,
                                                   uint32_t K, uint64_t sam, uint64_t sar, uint64_t sbr,
                                                   uint64_t sbn, uint64_t scm, uint64_t scn, uint32_t mtiles,
-                                                  uint32_t tiles) {
+                                                  uint32_t tiles, uint32_t blocks) {
     constexpr int TM = 16 * MH, TN = 16 * NH;
     // two chunks of both operands, or the staged results
     constexpr int LDS = 2 * kRT * (TM + TN) * 4 > TM * TN * 4 ? 2 * kRT * (TM + TN) * 4 : TM * TN * 4;
     __shared__ float4 lds[LDS];
+    const uint32_t bid = blockIdx.y * gridDim.x + blockIdx.x;
+    if (bid >= blocks) return;
     // tiles of one mode group are neighbours, and each XCD gets a contiguous
     // part of the list: the tiles that read the same operands, and the mode
     // groups that share their 128-byte lines, meet in one L2
-    const uint32_t u = bfly_dev::xcd_window(blockIdx.x, gridDim.x, gridDim.x >= 8 ? gridDim.x / 8 : 1);
+    const uint32_t u = bfly_dev::xcd_window(bid, blocks, blocks >= 8 ? blocks / 8 : 1);
     const uint32_t tile = u % tiles, k0 = u / tiles * kKT;
     const uint32_t m0 = (tile % mtiles) * TM, n0 = (tile / mtiles) * TN;
     const bool edge = m0 + TM > M || n0 + TN > N || k0 + kKT > K || R % kRT != 0;  // uniform
@@ -292,9 +295,12 @@ hipError_t launch_mix(const float2* A, const float2* B, float2* C, uint32_t M, u
     const uint32_t kt = (K + kKT - 1) / kKT, mt = (M + 16 * MH - 1) / (16 * MH), nt = (N + 16 * NH - 1) / (16 * NH);
     const uint64_t blocks = (uint64_t)kt * mt * nt;
     if (blocks == 0 || blocks > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    // a grid dimension holds less than 2^32 threads: 2^23 workgroups of 512
+    // (one row, column and channel of 2^26 modes) take a second one
+    const uint32_t gx = (uint32_t)(blocks < kMaxGridX ? blocks : kMaxGridX), gy = (uint32_t)((blocks + gx - 1) / gx);
     auto go = [&](auto v, auto cj) {
-        hipLaunchKernelGGL((k_mix<MH, NH, decltype(v)::value, decltype(cj)::value>), dim3((unsigned)blocks),
-                           dim3(kThreads), 0, s, A, B, C, M, N, R, K, sam, sar, sbr, sbn, scm, scn, mt, mt * nt);
+        hipLaunchKernelGGL((k_mix<MH, NH, decltype(v)::value, decltype(cj)::value>), dim3(gx, gy), dim3(kThreads), 0, s,
+                           A, B, C, M, N, R, K, sam, sar, sbr, sbn, scm, scn, mt, mt * nt, (uint32_t)blocks);
     };
     auto pick = [&](auto v) {
         if (conj == 0) go(v, std::integral_constant<int, 0>{});
