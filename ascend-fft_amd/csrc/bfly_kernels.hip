@@ -918,7 +918,20 @@ hipError_t launch_real(int kind, const float* in, float* out, const float2* tw, 
                 if (kind == 1 && bins <= (uint32_t)(PlanOf<I>::N / PlanOf<I>::RL))
                     return modes(&k_r2c_modes_lt<I>, rm[0], bins, stride, adj);
             if (kind == 2 && bins <= 2u * T) return modes(&k_c2r_modes_lt<I, 2>, rm[1], scale, bins, stride, adj);
-            if (kind == 2 && bins <= 4u * T) return modes(&k_c2r_modes_lt<I, 4>, rm[2], scale, bins, stride, adj);
+            // Four of the sixteen inputs: while rows and spectra are few, and
+            // where they are many; between, the full kernel is faster (n/8
+            // bins, pruned against full: 4096 x 1536 8.6 against 9.6 us, x 2048
+            // 12.3 against 11.5, x 4096 22.0 against 20.7, x 4608 23.5 against
+            // 24.5, x 8192 38.2 against 41.5; 2048 x 6144 15.6 against 16.0,
+            // 1024 x 8192 10.9 against 11.1).  512 points then pay for more
+            // than three inputs' bins (x 65536, 33 bins 41.6 against 38.5, 48
+            // bins 37.4 against 38.9).
+            constexpr int M = PlanOf<I>::N;
+            const uint64_t points = 2ull * M * batch;
+            const bool few = points <= (M == 1024 ? 3u << 22 : M == 512 ? 1u << 23 : 3u << 21);
+            const bool many = M == 256 ? points >= (7u << 21) && bins >= 3u * T : points > (1u << 24);
+            if (kind == 2 && bins <= 4u * T && (few || many))
+                return modes(&k_c2r_modes_lt<I, 4>, rm[2], scale, bins, stride, adj);
         }
         if (variant == BFLY_VARIANT_STREAM_LT) {
             const void* f = kind == 1 ? reinterpret_cast<const void*>(&k_r2c_stream_lt<I>)
