@@ -326,10 +326,7 @@ int bfly_c2c_ex(const float* in, float* out, uint32_t n, uint32_t batch, int sig
 int bfly_c2c_scaled(const float* in, float* out, uint32_t n, uint32_t batch, int sign, float scale,
                     const float* table, void* work, void* stream) {
     if (!std::isfinite(scale)) return BFLY_ERR_SHAPE;
-    // the variant whose last store applies the scale (AUTO above 4096; see
-    // bfly_host::scaled_variant)
-    const int variant = n <= (uint32_t)bfly_plan::kMaxLocalN ? BFLY_VARIANT_STREAM_LT : BFLY_VARIANT_AUTO;
-    return c2c_checked(in, out, n, batch, sign, variant, table, work, stream, scale);
+    return c2c_checked(in, out, n, batch, sign, bfly_host::scaled_variant(n), table, work, stream, scale);
 }
 
 int bfly_c2c(const float* in, float* out, uint32_t n, uint32_t batch, int sign,

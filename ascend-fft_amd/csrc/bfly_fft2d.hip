@@ -59,19 +59,20 @@ struct ColView {
 };
 
 // Rows that start on 128-byte lines: a run of 16 or more columns then covers
-// whole lines and takes the streaming hint (512 x 1024 x 32: 51.0 us against
-// 53.3 without it).  Other rows share every line with the neighbouring
-// columns' workgroup, which the L2 serves and merges only without the hint
-// (512 x 1001 x 24, windows of 8: 50.8 us against 76.4 with it).
+// whole lines and takes the streaming hint (512 x 1024 x 32: 48.1 us against
+// 52.1 without it, 256 x 1024 x 64 46.7 against 49.0).  Other rows share every
+// line with the neighbouring columns' workgroup, which the L2 serves and merges
+// only without the hint (256 x 1001 x 48 42.2 us against 73.1 with it, 1024 x
+// 1001 x 12 52.1 against 80.0).
 bool on_lines(const void* in, const void* out) {
     return (reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 128 == 0;
 }
 bool line_aligned(const void* in, const void* out, uint32_t ncols) { return ncols % 16 == 0 && on_lines(in, out); }
 
-// Units per XCD window (xcd_window) of the column kernels.  Sweep 1 / 2 / 4 /
-// 8 / 16 / 64 of the 16-point kernel: 512 x 1001 x 24 66.6 / 58.3 / 53.1 /
-// 50.8 / 50.4 / 54.3 us, 256 x 1024 x 64 55.3 / 55.1 / 54.4 / 51.3 / 48.9 us
-// (1 .. 16), 64 x 1001 x 200 53.5 / 49.2 / 46.0 / 44.6 / 42.6 / 42.6.
+// Units per XCD window (xcd_window) of k_cols.  Sweep 1 / 2 / 4 / 8 / 16 / 32 /
+// 64: 256 x 1001 x 48 66.3 / 55.5 / 48.4 / 44.0 / 42.2 / 41.0 / 41.7 us, 64 x
+// 1001 x 200 49.8 / 45.4 / 43.0 / 41.8 / 41.1 / 40.5 / 40.4, 256 x 1024 x 64 49.8 /
+// 49.4 / 48.3 / 47.0 / 46.6 / 46.7 / 46.9.
 constexpr uint32_t kColWindow = 4;  // log2
 constexpr uint32_t kAutoWindow = ~0u;
 
@@ -282,7 +283,13 @@ hipError_t launch_cols_wide(const float2* in, float2* out, const float2* tc, uin
     const int own = grid.own && on_line;
     const int in_hint = aligned || own;
     const int out_hint = (own && !aligned) || (aligned && (L == 512 || (L == 1024 && (WG < 1024 || blocks >= 512)) || (L == 2048 && WG == 512)));
-    // (log2 of the window)
+    // Windows (log2): 32 for rows off the lines, the best of 1 .. 64 at 512 x
+    // 1001 x 24 (58.9 us at 1, 49.6 at 8, 47.7 at 32, 49.8 at 64), 1024 x 1001 x
+    // 12 (68.6, 54.4, 52.2, 53.7), 2048 x 999 x 6 and 4096 x 333 x 9.  On the
+    // lines they matter less: 1024-thread groups of narrow 1024-point matrices
+    // take 64 (1024 x 256 x 64 52.3 us at 1, 51.4 at 32, 49.8 at 64), 4096
+    // points lose 25 % without (4096 x 1024 x 4 89.7 at 1, 66.5 at 16, 71.2 at
+    // 32), the others are equal within 2 % from 4.
     const uint32_t win = !aligned ? 5 : WG == 1024 ? (L == 1024 && ncols <= 256 ? 6 : 5) : WG == 512 && L < 2048 ? 5 : 2;
     if (sign < 0)
         hipLaunchKernelGGL((k_cols_wide<L, -1, WG>), dim3(blocks), dim3(WG), 0, s, in, out, tc, ncols, Divider(ncols), total, per,

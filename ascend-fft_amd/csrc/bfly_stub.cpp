@@ -228,7 +228,7 @@ int bfly_c2c_scaled(const float* in, float* out, uint32_t n, uint32_t batch, int
                     const float* table, void* work, void* stream) {
     if (!std::isfinite(scale)) return BFLY_ERR_SHAPE;
     if (!bfly_supported(BFLY_KIND_C2C, n)) return BFLY_ERR_SHAPE;
-    return bfly_c2c_ex(in, out, n, batch, sign, bfly_host::scaled_variant(n, batch), table, work, stream);
+    return bfly_c2c_ex(in, out, n, batch, sign, bfly_host::scaled_variant(n), table, work, stream);
 }
 int bfly_c2c_fwd(const float* in, float* out, uint32_t n, uint32_t batch, const float* table, void* work,
                  void* stream) {

@@ -297,8 +297,8 @@ int auto_kernel(uint32_t n, uint32_t batch) {
     return auto_variant(n, batch);
 }
 
-int scaled_variant(uint32_t n, uint32_t batch) {
-    return n <= (uint32_t)bfly_plan::kMaxLocalN ? BFLY_VARIANT_STREAM_LT : auto_variant(n, batch);
+int scaled_variant(uint32_t n) {
+    return n <= (uint32_t)bfly_plan::kMaxLocalN ? BFLY_VARIANT_STREAM_LT : BFLY_VARIANT_AUTO;
 }
 
 // Real transforms, once the batch fills several rounds of resident

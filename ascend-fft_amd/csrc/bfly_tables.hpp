@@ -100,10 +100,9 @@ struct PipeShape {
 int check_pipelined(int kind, int sign, int variant, const void* host_in, const void* host_out, uint32_t n,
                     uint32_t batch, const void* table, const void* dev_in, const void* dev_out, const void* work,
                     uint32_t chunk_rows, PipeShape* shape);
-// The public variant nearest to what bfly_c2c_scaled runs, one whose last
-// store applies the scale: the LDS-twiddle streaming kernel up to n = 4096,
-// AUTO's choice above.
-int scaled_variant(uint32_t n, uint32_t batch);
+// The variant bfly_c2c_scaled runs, one whose last store applies the scale: the
+// LDS-twiddle streaming kernel up to n = 4096, AUTO above.
+int scaled_variant(uint32_t n);
 
 // Guards of bfly_mode_mix: op 0..2, non-null 8-byte aligned operands, every
 // size >= 1, an output overlapping neither input, a grid that fits.

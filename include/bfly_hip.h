@@ -205,7 +205,8 @@ BFLY_API int bfly_c2c_scaled(const float* in, float* out, uint32_t n, uint32_t b
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): same
  * arguments minus `work`, same kernels, same results bit for bit.  No
  * counterpart in the reference.  The four-step chain's intermediate (the
- * only scratch a C2C uses: n > 16384, and 16384 with batch < 160) lives in a
+ * only scratch a C2C uses: n > 16384, counted at 32768 whichever kernel runs,
+ * and 16384 with batch < 160) lives in a
  * static device array of BFLY_NOALLOC_SCRATCH_BYTES per GPU, held until the
  * process ends; a shape whose intermediate (8 n batch bytes) does not fit
  * returns BFLY_ERR_SCRATCH (at 64 MiB: n * batch <= 8388608, e.g. 65536 x
@@ -228,13 +229,16 @@ BFLY_API int bfly_c2c_noalloc(const float* in, float* out, uint32_t n, uint32_t 
  * (config/test_matrix.json:94-99).  `table_rows` is the device copy of
  * bfly_table_fill(BFLY_KIND_C2C, n2), `table_cols` of bfly_fft2d_table_fill(n1);
  * `work` holds bfly_fft2d_workspace_bytes(n1, n2, batch) bytes.  Two HBM
- * round trips up to n1 = 2048, three at 4096. */
+ * round trips; three at n1 = 4096 with fewer than 1024 columns (n2 * batch). */
 /* Strided 1-D C2C along the first axis of `batch` row-major [n][ncols]
  * arrays (element stride ncols, adjacent transforms): X[k][c] = sum_j
  * x[j][c] e^{sign 2 pi i j k / n}; n a power of two in [16, 4096], any
- * ncols >= 1.  The column pass of bfly_fft2d on its own: one HBM round trip
- * up to n = 2048, two at 4096 through `work`
- * (bfly_c2c_columns_workspace_bytes; NULL allowed when that is 0).
+ * ncols >= 1.  The column pass of bfly_fft2d on its own: one HBM round trip;
+ * two through `work` at n = 4096 with fewer than 1024 columns (ncols * batch;
+ * the workspace of bfly_c2c_columns_workspace_bytes is asked for at 4096 in
+ * either case; NULL allowed when that is 0).  Kernels differ by the number of
+ * columns and by whether the buffers and rows start on 128-byte lines, so the
+ * last bits of a column may too (from n = 512).
  * `table_cols` is the device copy of bfly_fft2d_table_fill(n).  No
  * counterpart in the reference (non-contiguous layouts are future work
  * there, config/test_matrix.json:94-99, 106). */
