@@ -11,8 +11,8 @@ namespace bfly_cols {
 // values), so that `own` accesses take the streaming hint as whole-line rows
 // do.  Numbered through the batch, 256 columns of 1-column matrices ended up in
 // one workgroup, and every line was two groups'.  16 x 1 x 256 2.2 us against
-// 5.2, 256 x 1 x 120 4.9 against 6.0, 512 x 1 x 120 5.6 against 11.1, 512 x 12 x
-// 400 9.3 against 11.4, 2048 x 8 x 300 19.1 against 25.2.  Below 2^20 points
+// 5.2, 256 x 1 x 120 4.9 against 6.0, 512 x 1 x 120 5.8 against 11.1, 512 x 12 x
+// 400 8.9 against 11.6, 2048 x 8 x 200 14.0 against 17.3.  Below 2^20 points
 // (8 MB) and on rows of under 32 bytes the hint costs (64 x 5 x 256 4.8 us
 // against 3.5, 256 x 1 x 4000 9.9 against 7.6); groups that leave lanes idle
 // then number columns through the batch when they are many (16 x 100 x 600 4.6
@@ -23,12 +23,16 @@ struct Share {
 };
 inline Share column_share(uint32_t C, uint32_t L, uint32_t ncols, uint32_t total) {
     auto up = [](uint32_t a, uint32_t b) { return (a + b - 1) / b; };
-    if (ncols > C) {  // 16 points load and store with nothing between: spread over the CUs (16 x 1000 x 4 2.7 -> 2.3 us)
+    if (ncols > C) {
+        // 16 points load and store with nothing between: spread over the CUs
+        // (16 x 1000 x 4 2.7 -> 2.3 us; 64 x 300 x 20 would take 4.2 instead of 3.9)
         const uint32_t even = up(total, 256) < 64 ? 64 : up(total, 256);
         return {L == 16 && even < C ? even : C, false};
     }
     const uint32_t mats = total / ncols, fit = C / ncols;
-    // rows of at least 64 columns (32 at 128 points, 16 at 256), or 768 and 2048 rows
+    // 8 matrices of 16 or 32 points, longer ones up to about 768 rows (64 x 1 x
+    // 600 in 1 / 4 / 12 matrices 5.2 / 4.2 / 3.9 us, 64 x 8 x 120 6.9 / 4.1 / 3.5),
+    // but no more than 64 columns; 2048 rows at 1024 points (1 x 120 7.5 against 10.1)
     uint32_t least = L <= 32 ? 8 : L < 512 ? 768 / L : 1;
     least = L < 512 ? (least < up(C < 64 ? C : 64, ncols) ? least : up(C < 64 ? C : 64, ncols))
                     : L == 1024 && ncols == 1 ? 2 : 1;
@@ -61,13 +65,14 @@ inline Grid column_grid(uint32_t C, uint32_t L, uint32_t ncols, uint32_t total, 
 // them and parked behind.  GUARD: the loads lie under a branch, so that the
 // first butterflies wait for all of them; without it they start on the first
 // arrivals.  Measured on whole groups, by workgroups (four fit a CU):
-//   first               up to 512, and 256 points above 1024 (64 x 1024 x 37
-//                       9.1 -> 7.2 us; 256 x 1024 x 64 48.3 -> 47.2)
+//   first               up to 512, and 256 points above 1024 (128 x 256 x 32
+//                       4.9 -> 4.6 us; 256 x 1024 x 64 48.3 -> 47.2)
 //   first, guarded      513 to 1024: the workgroups of a CU no longer load all
 //                       at once (32 x 512 x 150 8.9 -> 7.5, 256 x 64 x 192
 //                       10.4 -> 8.8)
-//   ahead               above 1024 at 16 to 64 points (32 x 1024 x 512 44.5 -> 43.6) and 257 to
-//                       512 at 64 and 128 (128 x 128 x 128 6.5 -> 6.25)
+//   ahead               above 1024 at 16 to 64 points (32 x 1024 x 512 44.5
+//                       -> 43.6), 257 to 512 at 64 and 128 (128 x 128 x 128
+//                       6.5 -> 6.25)
 //   ahead, guarded      above 2560 at 128 points (128 x 2048 x 64 45.6 -> 44.7)
 enum Order { kFirst, kFirstGuard, kAhead, kAheadGuard };
 inline Order whole_order(int L, uint32_t blocks) {  // blocks: in 256 threads
