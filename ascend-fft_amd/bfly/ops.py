@@ -199,7 +199,8 @@ def fft2_raw(x: torch.Tensor, out: torch.Tensor, n1: int, n2: int, batch: int, s
     rc = lib.bfly_fft2d(x.data_ptr(), out.data_ptr(), n1, n2, batch, sign,
                         table(_lib.KIND_C2C, n2, x.device).data_ptr(), table2d_cols(n1, x.device).data_ptr(),
                         work.data_ptr(), _stream(x))
-    _lib.check(rc, f"bfly_fft2d(n1={n1}, n2={n2}, batch={batch}, sign={sign})")
+    if rc:
+        _lib.check(rc, f"bfly_fft2d(n1={n1}, n2={n2}, batch={batch}, sign={sign})")
 
 
 def fft_columns(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
@@ -220,7 +221,8 @@ def fft_columns(x: torch.Tensor, sign: int = -1) -> torch.Tensor:
     rc = lib.bfly_c2c_columns(x.data_ptr(), out.data_ptr(), n, ncols, batch, sign,
                               table2d_cols(n, x.device).data_ptr(), work.data_ptr() if work is not None else None,
                               _stream(x))
-    _lib.check(rc, f"bfly_c2c_columns(n={n}, ncols={ncols}, batch={batch}, sign={sign})")
+    if rc:
+        _lib.check(rc, f"bfly_c2c_columns(n={n}, ncols={ncols}, batch={batch}, sign={sign})")
     return out
 
 
@@ -250,7 +252,8 @@ def _real(kind: int, src: torch.Tensor, dst: torch.Tensor, n: int, batch: int, b
     rc = _lib.hip().bfly_real_ex(kind, src.data_ptr(), dst.data_ptr(), n, batch, bins, stride,
                                  _lib.VARIANT_AUTO, _lib.REAL_ADJOINT if adjoint else 0, tab.data_ptr(),
                                  _stream(src))
-    _lib.check(rc, f"{what}(n={n}, batch={batch}, bins={bins}, adjoint={adjoint})")
+    if rc:
+        _lib.check(rc, f"{what}(n={n}, batch={batch}, bins={bins}, adjoint={adjoint})")
 
 
 def rfft(x: torch.Tensor, adjoint: bool = False) -> torch.Tensor:
@@ -332,7 +335,8 @@ def mode_mix(op: int, a: torch.Tensor, b: torch.Tensor, batch: int, c_in: int, c
     a, b = plain(a), plain(b)
     rc = _lib.hip().bfly_mode_mix(op, a.data_ptr(), b.data_ptr(), out.data_ptr(), batch, c_in, c_out, modes,
                                   _stream(a))
-    _lib.check(rc, f"bfly_mode_mix(op={op}, batch={batch}, c_in={c_in}, c_out={c_out}, modes={modes})")
+    if rc:
+        _lib.check(rc, f"bfly_mode_mix(op={op}, batch={batch}, c_in={c_in}, c_out={c_out}, modes={modes})")
     return out
 
 

@@ -31,7 +31,7 @@ class MixModes(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, xm: torch.Tensor, w: torch.Tensor):
-        xm, w = ops.plain(xm.contiguous()), ops.plain(w.contiguous())
+        xm, w = xm.contiguous(), w.contiguous()
         B, C_in, K = xm.shape
         if w.shape[0] != C_in or w.shape[2] != K:
             raise ValueError(f"weights {tuple(w.shape)} do not match modes {tuple(xm.shape)}")
@@ -43,7 +43,7 @@ class MixModes(torch.autograd.Function):
     def backward(ctx, gy: torch.Tensor):
         xm, w = ctx.saved_tensors
         B, C_in, C_out, K = ctx.dims
-        gy = ops.plain(gy.contiguous())  # autograd hands over lazy conjugates
+        gy = gy.contiguous()
         gx = gw = None
         if ctx.needs_input_grad[0]:
             gx = ops.mode_mix(_lib.MIX_GRAD_INPUT, gy, w, B, C_in, C_out, K)

@@ -13,10 +13,11 @@ namespace bfly_cols {
 // one workgroup, and every line was two groups'.  16 x 1 x 256 2.2 us against
 // 5.2, 256 x 1 x 120 4.9 against 6.0, 512 x 1 x 120 5.8 against 11.1, 512 x 12 x
 // 400 8.9 against 11.6, 2048 x 8 x 200 14.0 against 17.3.  Below 2^20 points
-// (8 MB) and on rows of under 32 bytes the hint costs (64 x 5 x 256 4.8 us
-// against 3.5, 256 x 1 x 4000 9.9 against 7.6); groups that leave lanes idle
-// then number columns through the batch when they are many (16 x 100 x 600 4.6
-// against 5.3).
+// (8 MB) the hint costs (64 x 5 x 256 4.8 us against 3.5), and where a wave
+// stores parts of lines (256 x 5 x 3730 18.5 against 14.8, 64 x 39 x 866 10.2
+// against 8.8; the 1024- and 2048-point kernels still gain from two lines on:
+// 2048 x 7 x 300 15.1 against 19.6); groups that leave lanes idle then number
+// columns through the batch when they are many (16 x 100 x 600 4.6 against 5.3).
 struct Share {
     uint32_t per;
     bool own;
@@ -39,7 +40,9 @@ inline Share column_share(uint32_t C, uint32_t L, uint32_t ncols, uint32_t total
     uint32_t k = up(mats, 256);
     k = k < least ? least : k;
     k = k < fit ? k : fit;
-    const bool own = ncols >= 4 && (uint64_t)total * L >= (1u << 20);
+    // values that a wave's instruction stores side by side
+    const uint32_t run = C < 64 ? 64 / C * ncols : ncols;
+    const bool own = (run % 16 == 0 || (L >= 1024 && run >= 32)) && (uint64_t)total * L >= (1u << 20);
     if (!own && 8 * k * ncols < 7 * C && up(mats, k) > 256) return {C, false};
     return {k * ncols, own};
 }

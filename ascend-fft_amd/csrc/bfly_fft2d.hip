@@ -122,6 +122,13 @@ __global__ __launch_bounds__(WG) void k_cols(const float2* __restrict__ in, floa
         mi = cv.unit.divide(blk, &col);
         col = col * C + c;
         active = !GUARD || col < cv.ncols;
+    } else if (cv.ncols % C == 0) {
+        // (never at a launch of this form, but with this test in front of them
+        // the loads of ragged groups are scheduled better: 32 x 2099 x 57 11.3 ->
+        // 10.9 us, 16 x 689 x 378 11.9 -> 11.6)
+        mi = cv.unit.divide(blk, &col);
+        col = col * C + c;
+        active = true;
     } else {
         const uint32_t f0 = blk * cv.per, f = f0 + c;
         active = (uint32_t)c < cv.per && f < cv.total;
@@ -391,19 +398,30 @@ hipError_t launch_cols(const float2* in, float2* out, const float2* tw, const fl
     };
     constexpr std::integral_constant<Order, kFirst> first{};
     constexpr std::integral_constant<Order, kFirstGuard> first_guard{};
-    if (!whole) {
-        // ragged groups: tables ahead, at 16 and 32 points guarded (16 x 1000
-        // x 400 22.5 us against 23.7, 256 x 1001 x 48 44.0 against 42.5 at
-        // 256); matrices by themselves as whole groups at their workgroup counts
-        constexpr std::integral_constant<Order, kAheadGuard> ahead_guard{};
-        constexpr std::integral_constant<Order, L <= 32 ? kAheadGuard : kAhead> ragged{};
-        if (grid.own && blocks * (WG / 256) > 512 && blocks * (WG / 256) <= 1024) pick(std::false_type{}, first_guard);
-        else if (L == 64 && split && blocks > 512) pick(std::false_type{}, ahead_guard);  // as below
-        else pick(std::false_type{}, ragged);
-        return hipGetLastError();
-    }
-    // (the split's passes: 4096 x 5 x 200 25.9 us against 27.2 tables first, 29.8 unguarded)
-    const Order order = split && blocks > 512 ? kAheadGuard : whole_order(L, blocks * (WG / 256));
+    if constexpr (!TW)  // (the split's first pass is 64 ncols wide: whole)
+        if (!whole) {
+            // the split's second pass: tables first from 16 columns (4096 x 16 x
+            // 40 17.6 -> 15.6 us, 4096 x 100 x 7 18.9 -> 17.3), else as the first
+            // (4096 x 5 x 200 27.0 -> 25.9)
+            if constexpr (L == 64)
+                if (split && (cv.ncols >= 16 || blocks > 256)) {
+                    if (cv.ncols >= 16 && blocks > 512) pick(std::false_type{}, first_guard);
+                    else if (cv.ncols >= 16) pick(std::false_type{}, first);
+                    else pick(std::false_type{}, std::integral_constant<Order, kAheadGuard>{});
+                    return hipGetLastError();
+                }
+            // ragged groups: tables ahead, at 16 and 32 points guarded (16 x
+            // 1000 x 400 22.5 us against 23.7, 256 x 1001 x 48 44.0 against 42.5
+            // at 256); matrices by themselves as whole groups at their counts
+            const uint32_t in256 = blocks * (WG / 256);
+            if (grid.own && in256 > 512 && in256 <= 1024) pick(std::false_type{}, first_guard);
+            else pick(std::false_type{}, std::integral_constant<Order, L <= 32 ? kAheadGuard : kAhead>{});
+            return hipGetLastError();
+        }
+    // (the split's passes: 4096 x 5 x 200 25.9 us against 27.2 tables first, 29.8
+    // unguarded; 4096 x 5 x 60 14.9 tables first, 15.2 ahead)
+    const Order order = !split ? whole_order(L, blocks * (WG / 256))
+                        : blocks > 512 ? kAheadGuard : blocks > 448 ? kAhead : kFirst;
     if constexpr (L <= 128)
         if (order == kAhead) {
             pick(std::true_type{}, std::integral_constant<Order, kAhead>{});
@@ -451,8 +469,10 @@ hipError_t column_pass(const float* in, float* out, uint32_t n1, uint32_t ncols,
             // whole-line rows in fewer column groups than the wide kernel
             // needs to fill the chip: 512 x 64 x 4 5.7 us against 6.3, 512 x
             // 64 x 128 11.6 against 12.7 (512 x 64 x 256: 26.4 against 23.1)
-            // (and narrower than a line: 512 x 8 x 1000 11.6 against 12.4)
-            if ((al && F < 12288) || ncols < 16) return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, on_line, sign, s);
+            // (and narrower than a line, while few or in groups that own their
+            // lines: 512 x 8 x 1000 11.6 against 12.4; 512 x 1 x 5587 21.5 against 20.4)
+            if ((al && F < 12288) || (ncols < 16 && (F <= 4096 || column_grid(16, 512, ncols, F, true, true).own)))
+                return launch_cols<idx(512), false, 512>(i2, o2, t1, nullptr, cv, on_line, sign, s);
             return launch_wide<512>(i2, o2, t1, ncols, F, al, on_line, rows_behind, sign, s);
         case 1024:
             // whole-line rows, more columns than 256-thread workgroups take in

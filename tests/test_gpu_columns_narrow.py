@@ -32,6 +32,10 @@ SHAPES = [
     # 256, 512 and 1024 threads of the 32-point kernel on narrow matrices
     (1024, 12, 50), (1024, 12, 200), (1024, 8, 800), (1024, 7, 300), (2048, 3, 400), (2048, 5, 200), (2048, 12, 150),
     (4096, 3, 350), (4096, 7, 150), (4096, 1, 1100),
+    # 2^20 points and more where a wave stores parts of lines; 512-point ones from 4096 columns
+    (256, 5, 900), (64, 39, 500), (512, 1, 5000), (512, 7, 600),
+    # the 4096-point split: second pass ragged of 16 columns and more in few and many workgroups, and of fewer
+    (4096, 20, 8), (4096, 100, 7), (4096, 5, 60), (4096, 5, 3), (4096, 7, 100),
     # 16 points, ragged: spread
     (16, 300, 20), (16, 999, 70)]
 
